@@ -295,14 +295,12 @@ struct PrefillArgs {
     uint16_t *out;          // [n, Hq, Q, D] contiguous
     int32_t *err;
     int32_t n_items;
-    int32_t group;          // Hq / kv_heads (waves per workgroup)
+    int32_t group;          // Hq / kv_heads
     int32_t qn;             // Q (query rows per item)
     int32_t window;
-    int32_t heads_per_wg;   // q heads of the group served by one workgroup (divides group)
-    int32_t key_parts;      // waves per head splitting every tile's keys (1, 2 or 4)
-    int32_t ring_groups;    // > 0: LDS DMA ring of key_parts * ring_groups 32-key stages (prefill_ring_ok)
-    int32_t q_blocks;       // 16-query blocks per workgroup sharing its staged tiles (1; 2 on the ring)
-    int32_t n_ksplit;       // key ranges per query block; > 1: partials to part_o / part_ml
+    int32_t row_waves;      // 32-row blocks (q heads x queries) per workgroup
+    int32_t key_parts;      // waves per row block, splitting the keys
+    int32_t n_ksplit;       // key ranges per row block; > 1: partials to part_o / part_ml
     float *part_o;          // [n, Hq, Q, n_ksplit, D] unnormalised outputs
     float2 *part_ml;        // [n, Hq, Q, n_ksplit] (running max in log2 units, sum)
     const PrefixMask *pmask;  // non-null: prefix-attention masks, indexed by slot
@@ -363,7 +361,7 @@ struct CopyRowsArgs {
     int64_t t0, t1, tr;                       // dst strides in bytes
 };
 
-// ---- launchers (kvrt_kernels.hip) ----------------------------------------
+// ---- launchers (kvrt_kernels.hip, kvrt_prefill.hip) ----------------------------------------
 hipError_t launch_append(const AppendArgs &a, int head_dim, int dtype, int grid_x, hipStream_t s);
 hipError_t launch_gather(const GatherArgs &a, int head_dim, int dtype, hipStream_t s);
 // Split-K attention over the view, then the merge kernel.
@@ -376,24 +374,8 @@ hipError_t launch_decode_mfma(const DecodeArgs &a, int head_dim, int dtype, int 
 hipError_t launch_decode_talker(const TalkerArgs &a, int head_dim, int rows_per_head, hipStream_t s);
 // Chunked-prefill attention on MFMA (bf16 CONTIG / RING / PAGED layers).
 hipError_t launch_prefill(const PrefillArgs &a, int head_dim, hipStream_t s);
-// Most q heads one prefill workgroup computes (one wave each); a larger GQA
-// group is served by several workgroups.
-constexpr int kPfMaxHeads = 8;
-// Most waves per head (key parts) a prefill workgroup's tile buffers allow:
-// each part needs its own 32-key sub-tile, double-buffered in LDS.
-constexpr int kPfKeys = 32;  // keys per LDS sub-tile of the prefill kernel
-constexpr int prefill_max_parts(int head_dim) { return head_dim >= 512 ? 1 : head_dim >= 256 ? 2 : 4; }
-// Shapes of the prefill's LDS DMA ring: bf16 CONTIG / RING rows of 128 or
-// 256 dims, key_parts (1 or 2) * kPfRingGroups unpadded 32-key stages (K and
-// V), one group of key_parts stages computed while the next is in flight
-// (deeper rings measured slower: their LDS costs workgroups per CU); at
-// head_dim 128 one or two 16-query blocks per workgroup.
-constexpr int kPfRingGroups = 2;
-constexpr bool prefill_ring_ok(int head_dim, int layout, int key_parts, int groups, int q_blocks = 1) {
-    return (head_dim == 128 || head_dim == 256) && layout != KVRT_LAYOUT_PAGED && groups == kPfRingGroups &&
-           (key_parts == 1 || key_parts == 2) && key_parts * groups * 32 * head_dim * 2 * 2 <= 128 * 1024 &&
-           (q_blocks == 1 || (q_blocks == 2 && head_dim == 128));
-}
+hipError_t launch_prefill_wide(const PrefillArgs &a, int head_dim, hipStream_t s);  // head_dim 256, 512
+constexpr int kPfKeys = 32;  // keys per staged block of the prefill kernel
 hipError_t launch_set_lens(const SetLenArgs &a, hipStream_t s);
 hipError_t launch_set_pages(int32_t *pt, int n, const int32_t *idx, const int32_t *val,
                             hipStream_t s);

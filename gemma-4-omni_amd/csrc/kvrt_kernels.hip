@@ -13,84 +13,9 @@
 //
 // Every memory-bound loop moves 16 B per lane with consecutive lanes on
 // consecutive addresses (one 1 KiB transaction per wave instruction).
-#include <type_traits>
-
-#include "kvrt_device.h"
-#include "kvrt_internal.h"
+#include "kvrt_wave.h"
 
 namespace kvrt {
-
-constexpr float kNegBig = -1.0e30f;  // running-max start; exp2(kNegBig - m) == 0
-// Lazy online softmax: a running max m (log2 units) moves only when a block's
-// max exceeds it by more than kRescaleSlack, so p = 2^(s - m) stays <= 2^8
-// and the accumulator rescale runs a few times per wave instead of on most
-// blocks. Exact: l and the accumulator always refer to the same m, and every
-// merge weights a partial by its own m.
-constexpr float kRescaleSlack = 8.0f;
-
-// Row number of position pos of a head on a PAGED page, in pool order
-// ((page, head, pos % rows)); -1 if the page is unmapped or out of the pool.
-// 32-bit arithmetic: the host keeps pool_pages below 2^24 and the pool's rows
-// below 2^31, so page * (kv_heads * rows) is a 24-bit product.
-__device__ __forceinline__ int page_row(const KVView &v, int page, int head, int pos) {
-    if (page < 0 || page >= v.pool_pages) return -1;
-    return (int)__umul24((unsigned)page, (unsigned)(v.kv_heads * v.rows)) + head * v.rows + (pos & (v.rows - 1));
-}
-
-// Element offset of the first element of row (slot, head, pos); -1 if the
-// page is unmapped or out of the pool.
-template <int LAYOUT>
-__device__ __forceinline__ int64_t row_offset(const KVView &v, int slot, int head, int pos, int D) {
-    if constexpr (LAYOUT == KVRT_LAYOUT_CONTIG) {
-        return slot * v.slot_stride + head * v.head_stride + (int64_t)pos * v.row_stride;
-    } else if constexpr (LAYOUT == KVRT_LAYOUT_RING) {
-        return slot * v.slot_stride + head * v.head_stride + (int64_t)(pos % v.rows) * v.row_stride;
-    } else {
-        const int lp = pos >> v.block_shift;
-        if (pos < 0 || lp >= v.pt_stride) return -1;
-        const int page = v.page_table[(int64_t)slot * v.pt_stride + lp];
-        const int row = page_row(v, page, head, pos);
-        return row < 0 ? -1 : (int64_t)row * D;
-    }
-}
-
-// Prefix-attention mask of a slot as a wave holds it: its length plen (0: no
-// mask; wave-uniform, in an SGPR) and, in every lane, mask word (lane & 15).
-// The record is read only when the launch carries masks, so launches without
-// them load nothing. Both values are waited for here, so callers issue this
-// next to their length load (one memory round trip for both) and before any
-// LDS DMA: the compiler does not count inline-assembly DMAs, and a wait it
-// placed for these loads inside a DMA-pipelined loop would drain the ring.
-__device__ __forceinline__ void load_prefix(const PrefixMask *pm, int slot, int lane, int &plen, uint32_t &pw) {
-    plen = 0;
-    pw = 0xffffffffu;
-    if (pm != nullptr) {
-        plen = __builtin_amdgcn_readfirstlane(pm[slot].len);
-        pw = pm[slot].bits[lane & (kPrefixWords - 1)];
-        asm volatile("" ::"v"(pw));  // the word is in its register from here on
-    }
-}
-// Mask bit of key position key (0 <= key < KVRT_MAX_PREFIX_MASK): the word
-// comes from the lane that holds it (ds_bpermute), so every lane of the wave
-// must call this together.
-__device__ __forceinline__ bool prefix_bit(uint32_t pw, int key) {
-    const uint32_t w = (uint32_t)__shfl((int)pw, (key >> 5) & (kPrefixWords - 1));
-    return ((w >> (key & 31)) & 1u) != 0;
-}
-// Mask bits of the 8 keys k0 .. k0 + 7 (k0 >= 0; bit j: key k0 + j passes
-// the mask of length plen), branch-free: the two words they span come from
-// the lanes that hold them, keys at or past plen pass. Every lane of the wave
-// must call this together.
-__device__ __forceinline__ uint32_t prefix_bits8(uint32_t pw, int k0, int plen) {
-    const int w = k0 >> 5;
-    const uint32_t lo = (uint32_t)__shfl((int)pw, w & (kPrefixWords - 1));
-    const uint32_t hi = (uint32_t)__shfl((int)pw, (w + 1) & (kPrefixWords - 1));
-    const uint32_t bits = (uint32_t)((((uint64_t)hi << 32) | lo) >> (k0 & 31)) & 0xffu;
-    const int past = plen - k0;  // keys j >= past are beyond the mask
-    const uint32_t open = past <= 0 ? 0xffu : past >= 8 ? 0u : (0xffu << past) & 0xffu;
-    return bits | open;
-}
-
 
 // Item of grid z-index z of a PAGED decode: order[] read as aligned words
 // through the scalar cache (a byte read is a vector load: one more memory
@@ -100,36 +25,6 @@ __device__ __forceinline__ int launch_item(const DecodeArgs &a, int z) {
     uint32_t w;
     __builtin_memcpy(&w, a.order + 4 * (z >> 2), 4);
     return (int)((w >> (8 * (z & 3))) & 0xffu);
-}
-
-// q = x / d and r = x % d for x >= 0 and a wave-uniform d > 0: a shift and a
-// mask when d is a power of two (a uniform branch), else the division.
-__device__ __forceinline__ void udivmod_uniform(int x, int d, int &q, int &r) {
-    if ((d & (d - 1)) == 0) {
-        q = x >> __builtin_ctz((unsigned)d);
-        r = x & (d - 1);
-    } else {
-        q = x / d;
-        r = x - q * d;
-    }
-}
-__device__ __forceinline__ int umod_uniform(int x, int d) {
-    int q, r;
-    udivmod_uniform(x, d, q, r);
-    return r;
-}
-
-// A wave's window of page-table entries: lane i holds the entry of logical
-// page win0 + i of the slot (-1 past the table).
-__device__ __forceinline__ int load_page_window(const KVView &v, int slot, int win0, int lane) {
-    const int lp = win0 + lane;
-    return lp < v.pt_stride ? v.page_table[(int64_t)slot * v.pt_stride + lp] : -1;
-}
-// Element offset of row pos of a head on a page; -1 if the page is unmapped
-// or out of the pool.
-__device__ __forceinline__ int64_t page_row_offset(const KVView &v, int page, int head, int pos, int D) {
-    const int row = page_row(v, page, head, pos);
-    return row < 0 ? -1 : (int64_t)row * D;
 }
 
 // Symmetric int8 quantisation of one (token, head) row whose D values are
@@ -476,49 +371,6 @@ __global__ __launch_bounds__(256) void gather_kernel(GatherArgs a) {
 // ---------------------------------------------------------------------------
 // decode attention (split-K)
 // ---------------------------------------------------------------------------
-// LDS DMA: global_load_lds_dwordx4 moves lane l's 16 bytes at g to LDS byte
-// M0 + 16 * l without passing through registers. It is issued from inline
-// assembly (the LDS address is an M0 operand the compiler sets up), so the
-// compiler neither tracks these loads nor inserts its own (all-or-nothing)
-// waits for them: the decode waits with explicit vmcnt waits — vector loads
-// complete in issue order, so vmcnt(N) means every DMA but the N most recent
-// has landed — and reads the LDS back only after such a wait.
-__device__ __forceinline__ void dma_load16(const void *g, uint32_t lds) {
-    asm volatile("global_load_lds_dwordx4 %0, off nt" ::"v"(g), "{m0}"(lds) : "memory");
-}
-// 4 bytes per lane, to LDS byte M0 + 4 * l.
-__device__ __forceinline__ void dma_load4(const void *g, uint32_t lds) {
-    asm volatile("global_load_lds_dword %0, off nt" ::"v"(g), "{m0}"(lds) : "memory");
-}
-// The same without the streaming hint, for tiles other workgroups read again.
-__device__ __forceinline__ void dma_load16_cached(const void *g, uint32_t lds) {
-    asm volatile("global_load_lds_dwordx4 %0, off" ::"v"(g), "{m0}"(lds) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void wait_vmem() {
-    static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-// Waits until at most n * STEP vector memory operations are outstanding,
-// n in [0, NMAX] (wave-uniform).
-template <int STEP, int NMAX>
-__device__ __forceinline__ void wait_vmem_steps(int n) {
-    if constexpr (NMAX > 0) {
-        if (n >= NMAX) {
-            wait_vmem<NMAX * STEP>();
-            return;
-        }
-        wait_vmem_steps<STEP, NMAX - 1>(n);
-    } else {
-        wait_vmem<0>();
-    }
-}
-__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-template <class T>
-__device__ __forceinline__ uint32_t lds_addr(const T *p) {
-    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) T *)p;
-}
-
 // LDS floats a decode workgroup needs for its cross-wave merge: the partials
 // of waves 1..3, when R * D is small enough to stage them.
 // Online merge of the partials sp = j, j + G, ... < n of one output element
@@ -1209,10 +1061,6 @@ __global__ __launch_bounds__(256) void decode_kernel(Args a) {
     }
 }
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef short s16x4_t __attribute__((ext_vector_type(4)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-
 __device__ __forceinline__ f32x4_t mfma16(uint4 a, uint4 b, f32x4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b),
                                                    c, 0, 0, 0);
@@ -1235,14 +1083,6 @@ __device__ __forceinline__ void lazy_rescale(float tmax, float &m, float &l, f32
         }
         m = tmax;
     }
-}
-
-// gfx950 LDS transpose read: in each group of 16 lanes, lane s gives the
-// address of 4 consecutive bf16; lane t = 4a + e receives element e of the
-// chunks of lanes a, a + 4, a + 8, a + 12.
-__device__ __forceinline__ uint2 lds_read_tr16(const uint16_t *p) {
-    const s16x4_t x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4_t __attribute__((address_space(3))) *)(p));
-    return __builtin_bit_cast(uint2, x);
 }
 
 // Split-K decode on MFMA for R = g*Q in {8, 16} query rows per kv head
@@ -2096,629 +1936,6 @@ __global__ __launch_bounds__(256) void merge_kernel(DecodeArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// chunked-prefill attention (MFMA)
-// ---------------------------------------------------------------------------
-// grid (n_ksplit * kv_heads * g / hw, n_items, ceil(Q / 16)), 64 * NW
-// threads with NW = 4 or 8 >= hw: workgroup (x, y, z) serves key range
-// x % n_ksplit of the hw q heads kvh*g + (b % (g/hw))*hw + j (wave j < hw,
-// b = x / n_ksplit, kvh = b / (g/hw)) of item y over the 16 query rows of
-// block ceil(Q / 16) - 1 - z (on the DMA ring with QB = 2: z over ceil(Q / 32)
-// pairs of blocks, waves hw .. 2 hw - 1 on the second block of the pair);
-// all NW waves stage each 32-key K/V tile into LDS (K row-major, V
-// transposed) and the hw computing waves share it. With PF the next tile's
-// global loads are issued into registers before the current tile is
-// computed, so their latency hides behind the MFMAs. Per tile and computing
-// wave:
-//   S^T (32 keys x 16 queries) = K Q^T      2 * D/32  v_mfma_f32_16x16x32_bf16
-//   online softmax per query column (fp32, exp2 domain)
-//   O^T (D x 16) += V^T P^T                 2 * D/16  v_mfma_f32_16x16x32_bf16
-// with P split into two bf16 terms for the second product and everything
-// accumulated in fp32. MFMA lane layouts (16x16x32): A[row l%16][k 8(l/16)+j],
-// B[k 8(l/16)+j][col l%16], D[row 4(l/16)+v][col l%16].
-
-// Key (within a tile) of row i of S^T block b. Chosen so that lane group G
-// (lanes 16G..16G+15) ends up with the scores of keys 8G..8G+7 across the two
-// blocks, which are exactly the keys of its B operand in V^T P^T.
-__device__ __forceinline__ int pf_key(int b, int i) { return 8 * (i >> 2) + 4 * b + (i & 3); }
-
-// Calls f(integral_constant<int, u>) for u = U .. N-1: register arrays
-// indexed by u stay in registers.
-template <int U, int N>
-struct StaticFor {
-    template <class F>
-    __device__ __forceinline__ static void run(F &&f) {
-        if constexpr (U < N) {
-            f(std::integral_constant<int, U>{});
-            StaticFor<U + 1, N>::run(f);
-        }
-    }
-};
-
-// Tile units: unit c = (row c / (D/8), 16 B segment c % (D/8)) of both the
-// K and the V tile, both staged row-major. Keys at or past kend read row
-// kclamp (a key of the cache, masked in the softmax).
-// Element offset of row kr of the tile at t0 (key t0 + kr; keys at or past
-// kend read row kclamp).
-template <int D, int LAYOUT>
-__device__ __forceinline__ int64_t pf_row_offset(const KVView &kv, int slot, int kvh, int t0, int kclamp, int kend,
-                                                 int kr, bool &bad) {
-    const int key = t0 + kr;
-    if constexpr (LAYOUT == KVRT_LAYOUT_CONTIG) {
-        // one multiply-add per row from the (slot, head) base
-        const int64_t base = (int64_t)slot * kv.slot_stride + (int64_t)kvh * kv.head_stride;
-        return base + (int64_t)(key < kend ? key : kclamp) * D;
-    } else if constexpr (LAYOUT == KVRT_LAYOUT_RING) {
-        // t0 % rows once per tile: rows of the tile wrap at most once
-        const int64_t base = (int64_t)slot * kv.slot_stride + (int64_t)kvh * kv.head_stride;
-        const int r0 = t0 % kv.rows, rs = kclamp % kv.rows;
-        int rk = r0 + kr;
-        rk = rk >= kv.rows ? rk - kv.rows : rk;
-        return base + (int64_t)(key < kend ? rk : rs) * D;
-    } else {
-        const int64_t off = row_offset<LAYOUT>(kv, slot, kvh, key < kend ? key : kclamp, D);
-        bad |= off < 0;
-        return off < 0 ? 0 : off;
-    }
-}
-
-template <int D, int LAYOUT, int TK>
-__device__ __forceinline__ void pf_fetch_unit(const KVView &kv, int slot, int kvh, int t0, int kclamp, int kend, int c,
-                                              u32x4_t &kx, u32x4_t &vx, bool &bad) {
-    constexpr int UNITS = TK * (D / 8);
-    const uint16_t *kg = static_cast<const uint16_t *>(kv.k);
-    const uint16_t *vg = static_cast<const uint16_t *>(kv.v);
-    const int cc = c < UNITS ? c : 0;
-    const int kr = cc / (D / 8), ks = cc % (D / 8);
-    const int64_t off = pf_row_offset<D, LAYOUT>(kv, slot, kvh, t0, kclamp, kend, kr, bad);
-    kx = *reinterpret_cast<const u32x4_t *>(kg + off + 8 * ks);
-    vx = *reinterpret_cast<const u32x4_t *>(vg + off + 8 * ks);
-}
-
-// LDS layout of a staged K or V tile: row r (key) at r * pf_pitch<D>() bf16,
-// its 16-B chunk k at chunk position k ^ pf_swz<D>(r). With D >= 128 the
-// rows carry 32 B of padding and chunks are XOR-swizzled by bits 3 and 4 of
-// the row, so that the 16 rows x 16 B of one S^T A-operand read and the 8 rows
-// x 32 B of one V^T transposed read of a half-wave fall on distinct banks
-// (64 banks of 4 B); D = 64 keeps 16 B of padding and no swizzle.
-template <int D>
-constexpr int pf_pitch() { return D >= 128 ? D + 16 : D + 8; }
-template <int D>
-__device__ __forceinline__ int pf_swz(int r) { return D >= 128 ? (((r >> 3) & 1) * 8) ^ ((r >> 4) & 1) : 0; }
-// Chunk swizzle of the unpadded DMA-ring stages (rows of D bf16, 16-B chunk c
-// of row r at c ^ pf_rswz(r), r < 32): bits 0, 1, 3 and 4 of the row move
-// chunk bits 1, 2, 3 and 0. With 64 banks of 4 B, the 16 rows x 16 B of one
-// S^T A-operand read (keys pf_key(b, 0..15)) land on 16 distinct 16-B bank
-// groups and the 8 rows x 2 chunks of a half-wave V^T transposed read on 16
-// (found by enumerating XOR maps of the row bits); bit 2 is unused, so rows
-// r and r + 4 (the two halves of a transposed read) share the swizzle.
-__device__ __forceinline__ int pf_rswz(int r) { return ((r & 3) << 1) | (((r >> 3) & 1) << 3) | ((r >> 4) & 1); }
-
-// EXACT: every thread's unit is in the tile (UNITS a multiple of the block),
-// so no lane is masked off: a branch here would make the compiler wait for
-// every outstanding load at its join, the next tile's prefetch included.
-template <int D, int TK, bool EXACT>
-__device__ __forceinline__ void pf_stage_unit(uint16_t *sk, uint16_t *sv, int c, const u32x4_t &kx, const u32x4_t &vx) {
-    constexpr int UNITS = TK * (D / 8);
-    constexpr int KP = pf_pitch<D>();
-    if (EXACT || c < UNITS) {
-        const int kr = c / (D / 8), ks = (c % (D / 8)) ^ pf_swz<D>(c / (D / 8));
-        *reinterpret_cast<u32x4_t *>(&sk[kr * KP + 8 * ks]) = kx;
-        *reinterpret_cast<u32x4_t *>(&sv[kr * KP + 8 * ks]) = vx;
-    }
-}
-
-// A whole tile of TK keys, KU units per thread: unit u of thread t is
-// c = t + u * blockDim (the rows of a tile of KS sub-tiles are consecutive).
-template <int D, int LAYOUT, int TK, int KU, int NT>
-__device__ __forceinline__ void pf_fetch(const KVView &kv, int slot, int kvh, int t0, int kclamp, int kend,
-                                         u32x4_t (&kreg)[KU], u32x4_t (&vreg)[KU], bool &bad) {
-    StaticFor<0, KU>::run([&](auto uc) {
-        constexpr int u = decltype(uc)::value;
-        pf_fetch_unit<D, LAYOUT, TK>(kv, slot, kvh, t0, kclamp, kend, threadIdx.x + u * NT, kreg[u], vreg[u], bad);
-    });
-}
-
-template <int D, int TK, int KU, int NT>
-__device__ __forceinline__ void pf_stage(uint16_t *sk, uint16_t *sv, const u32x4_t (&kreg)[KU], const u32x4_t (&vreg)[KU]) {
-    constexpr bool EXACT = (TK * (D / 8)) % NT == 0;
-    StaticFor<0, KU>::run([&](auto uc) {
-        constexpr int u = decltype(uc)::value;
-        pf_stage_unit<D, TK, EXACT>(sk, sv, threadIdx.x + u * NT, kreg[u], vreg[u]);
-    });
-}
-
-template <int D, int LAYOUT, int NW, bool PF, int KS, int G = 0, int QB = 1>
-__global__ __launch_bounds__(64 * NW) void prefill_kernel(PrefillArgs a) {
-    constexpr int KP = pf_pitch<D>();  // K / V tile row pitch (bf16)
-    constexpr int TK = kPfKeys * KS;   // keys per iteration: KS sub-tiles of 32
-    constexpr int UNITS = TK * (D / 8);  // 16-B units of a K (or V) tile
-    constexpr int KU = (UNITS + 64 * NW - 1) / (64 * NW);  // units per thread
-    constexpr int PD = KU <= 2 ? 4 : 2;                      // tiles in flight with PF
-    // two K/V tile buffers, so tile t + 1 is staged while tile t is computed
-    constexpr int NBUF = 2;
-    constexpr int SUB = kPfKeys * KP;   // bf16 elements of one 32-key sub-tile
-    constexpr int TILE = KS * SUB;      // bf16 elements of one K (or V) tile buffer
-    // G > 0: the LDS DMA ring (bf16 CONTIG / RING, D 128 / 256): NS = KS * G
-    // unpadded, swizzled 32-key stages (pf_rswz), G - 1 groups of KS in flight
-    constexpr bool RG = G > 0;
-    // QB = 2: two consecutive 16-query blocks share the workgroup's staged
-    // tiles (half the tile traffic and DMA instructions per block)
-    static_assert(QB == 1 || (QB == 2 && RG && D == 128), "query-block pairs: DMA ring, head_dim 128");
-    constexpr int NS = KS * (RG ? G : 1);
-    constexpr int RSUB = kPfKeys * D;   // bf16 elements of one ring stage (K or V)
-    constexpr int LDS_ELEMS = RG ? NS * RSUB : NBUF * TILE;
-    static_assert(PF || KS == 1, "the LDS DMA path stages 32-key tiles");
-    static_assert(!RG || (PF && (D == 128 || D == 256) && LAYOUT != KVRT_LAYOUT_PAGED && G >= 2 &&
-                          (D / 8) % NW == 0), "DMA ring: bf16 CONTIG / RING, D 128 / 256");
-    // the KS - 1 upper parts' accumulators fit the tile buffers for the final combine
-    static_assert((KS - 1) * (NW / KS) * 16 * D * 4 <= LDS_ELEMS * 2, "part combine fits LDS");
-    static_assert((KS - 1) * (NW / KS) * 16 * 8 <= LDS_ELEMS * 2, "part (m, l) fit LDS");
-    __shared__ __align__(16) uint16_t sk[LDS_ELEMS];
-    __shared__ __align__(16) uint16_t sv[LDS_ELEMS];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int col = lane & 15, grp = lane >> 4;
-    const int hw = a.heads_per_wg;
-    int nhb, rem;
-    udivmod_uniform(a.group, hw, nhb, rem);
-    // Wave w computes head w % hw over key part (w / hw) % KS of the
-    // workgroup's query block w / (hw KS): within every tile, part p takes
-    // the 32-key sub-tile p, and the parts' accumulators are combined at the
-    // end (KS > 1 puts 2 or 4 waves on one head and query block without
-    // staging any tile twice; QB > 1 puts QB blocks on the same tiles).
-    int hidx, wrest;
-    udivmod_uniform(wave, hw, wrest, hidx);
-    const int part = KS > 1 ? wrest % KS : 0;
-    const int qsub = QB > 1 ? wrest / KS : 0;  // this wave's block of the workgroup's QB
-    // Grid (head part x key range, item, query blocks): workgroups start in
-    // linear id order, so the query blocks are the most significant and run
-    // last blocks first. Without a window the last blocks see the most keys:
-    // the longest workgroups start first and the grid's tail is short ones.
-    const int nks = a.n_ksplit;
-    int by, ks;
-    udivmod_uniform(blockIdx.x, nks, by, ks);
-    const int item = blockIdx.y;
-    const int qb = gridDim.z - 1 - blockIdx.z;
-    int kvh, hb;
-    udivmod_uniform(by, nhb, kvh, hb);
-    const int hkv = a.kv.kv_heads;
-    const int g = a.group, hq = hkv * g;
-    const bool computes = wave < hw * KS * QB;
-    const int head = kvh * g + hb * hw + (computes ? hidx : 0);
-    const int slot = a.slots[item];
-    const int L = a.len.lens[(int64_t)slot * a.len.stride + a.len.offset];
-    int plen;  // prefix-attention mask of the slot
-    uint32_t pw;
-    load_prefix(a.pmask, slot, lane, plen, pw);
-    const int Qn = a.qn;
-    const int qrow0 = (qb * QB + qsub) * 16;   // this wave's block
-    const int base_pos = L - Qn;               // position of query row 0
-    const int qr = qrow0 + col;                // this lane's query row (S^T / O^T column)
-    const bool qvalid = computes && qr < Qn;
-    const int pq = base_pos + qr;
-    const int lo_q = a.window > 0 ? pq - a.window + 1 : 0;
-    // the workgroup's keys: up to its last block's last query, from its first
-    // block's first query's window; with a key split, part ks of them in
-    // whole tiles
-    int kend = base_pos + min(Qn, (qb + 1) * QB * 16);
-    int kstart = a.window > 0 ? max(0, base_pos + qb * QB * 16 - a.window + 1) : 0;
-    // this wave's own block's keys (QB > 1: a step outside them is skipped)
-    const int wkend = base_pos + min(Qn, qrow0 + 16);
-    const int wkstart = a.window > 0 ? max(0, base_pos + qrow0 - a.window + 1) : 0;
-    const bool wlive = computes && qrow0 < Qn;
-    const int kblock = kstart;  // the block's first key: a row of the cache
-    if (nks > 1) {
-        const int span = (kend - kstart + nks - 1) / nks;
-        const int part = (span + kPfKeys - 1) / kPfKeys * kPfKeys;
-        const int k0 = kstart + ks * part;
-        kend = min(kend, k0 + part);
-        kstart = min(k0, kend);
-    }
-    // Rows fetched past the range read row kclamp and are masked: the range's
-    // first key, or the block's first key when the split left this range
-    // empty (kstart == kend can be one past the slot's last row, on a page
-    // not mapped or, in CONTIG storage, past the layer's rows)
-    const int kclamp = kstart < kend ? kstart : kblock;
-
-    // Q^T as the B operand: lane (col, grp) holds d = 32c + 8grp .. +7 of query qr.
-    uint4 qop[D / 32];
-    {
-        const uint16_t *qp = a.q + (((int64_t)item * hq + head) * Qn + (qvalid ? qr : 0)) * D + 8 * grp;
-#pragma unroll
-        for (int c = 0; c < D / 32; ++c)
-            qop[c] = qvalid ? *reinterpret_cast<const uint4 *>(qp + 32 * c) : make_uint4(0, 0, 0, 0);
-    }
-    float m = kNegBig, l = 0.f;  // running max (uniform per query) and this lane's partial sum
-    f32x4_t o[D / 16];
-#pragma unroll
-    for (int b = 0; b < D / 16; ++b) o[b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    bool bad = false;
-    // keys this lane's query sees in the block's range: [klo, khi] (none if
-    // the lane has no query)
-    const int khi = qvalid ? min(kend - 1, pq) : -1;
-    const int klo = lo_q;
-
-    // The MFMA work on the tile staged in LDS, keys t0 .. t0 + 31.
-    // V^T operand rows through gfx950's LDS transpose read: in each group of
-    // 16 lanes, lane s points at key row 8*grp + s/4 (+4 for the second
-    // read), dims 4*(s%4) .. +3 of the 16-dim block; lane t = 4a + e then
-    // receives dim 4a + e of key rows 8*grp + j, j = 0..3, i.e. A[d][k].
-    // (swizzle: row 8grp + ... has bit 3 = grp & 1 and bit 4 = grp >> 1, so
-    // chunk (col&3)/2 + 2*b sits at ((col&3)/2 ^ (grp >> 1)) + 2*(b ^ 4*(grp & 1)):
-    // blocks b with bit 2 clear read 64 elements further when grp is odd, the
-    // others 64 nearer)
-    const int vd = D >= 128 ? (grp & 1) * 64 : 0;
-    // this wave's sub-tile of every tile buffer (key part `part`)
-    const uint16_t *sk_w = sk + part * SUB;
-    const uint16_t *sv_base =
-        &sv[part * SUB + (8 * grp + (col >> 2)) * KP + 8 * (((col & 3) >> 1) ^ (D >= 128 ? grp >> 1 : 0)) +
-            4 * (col & 1)];
-    const uint16_t *sv_lo = sv_base + vd, *sv_hi = sv_base - vd;
-    auto read_vt = [&](const uint16_t *p) __attribute__((always_inline)) {
-        typedef short v4s_t __attribute__((ext_vector_type(4)));
-        const v4s_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (v4s_t __attribute__((address_space(3))) *)(p));
-        const v4s_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (v4s_t __attribute__((address_space(3))) *)(p + 4 * KP));
-        const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
-        return make_uint4(l2.x, l2.y, h2.x, h2.y);
-    };
-    // The work on one staged 32-key tile: kop(b, c) is key row pf_key(b, col)'s
-    // A operand of reduction step c, vop(b) the V^T operand of dims 16b ..
-    // 16b + 15 (both read from LDS).
-    auto tile_core = [&](int t0, auto kop, auto vop) __attribute__((always_inline)) {
-        // every key of the tile visible to all 16 queries of the block (the
-        // block's first query sees up to its own position, the last one's
-        // window starts at or before t0): no per-key mask
-        const bool all_visible = qrow0 + 16 <= Qn && t0 + kPfKeys - 1 <= base_pos + qrow0 &&
-                                 (a.window == 0 || t0 >= base_pos + qrow0 + 15 - a.window + 1) && t0 >= plen;
-        // S^T blocks: rows = keys pf_key(b, i), cols = queries
-        f32x4_t s[2];
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            s[b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-            // chunk grp + 4c of key row kr sits at (grp ^ s0) + 4 * (c ^ 2 s3)
-            // (s0, s3: bits 4 and 3 of kr): slices c with bit 1 clear read 64
-            // elements further when s3 is set, the others 64 nearer
-#pragma unroll
-            for (int c = 0; c < D / 32; ++c) s[b] = mfma16(kop(b, c), qop[c], s[b]);
-        }
-        // mask and scale; this lane holds keys 8grp .. 8grp+7 of the tile.
-        // Tiles every query sees whole take no per-key test; the others a
-        // branch-free one: key in [klo, khi] and passing the prefix mask.
-        float sc[8];
-        float tmax = -INFINITY;
-        if (all_visible) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                sc[j] = (j < 4 ? s[0][j] : s[1][j - 4]) * a.scale_log2;
-                tmax = fmaxf(tmax, sc[j]);
-            }
-        } else {
-            // bit j of vis8: key k0 + j lies in [klo, khi] and passes the
-            // prefix mask; one bit test per key
-            const int k0 = t0 + 8 * grp;
-            const uint32_t pvis = t0 < plen ? prefix_bits8(pw, k0, plen) : 0xffu;
-            const int nhi = min(max(khi - k0 + 1, 0), 8), nlo = min(max(klo - k0, 0), 8);
-            const uint32_t vis8 = ((1u << nhi) - 1u) & ~((1u << nlo) - 1u) & pvis;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                sc[j] = (vis8 & (1u << j)) != 0 ? (j < 4 ? s[0][j] : s[1][j - 4]) * a.scale_log2 : -INFINITY;
-                tmax = fmaxf(tmax, sc[j]);
-            }
-        }
-        tmax = pair<OpMax, 32>(pair<OpMax, 16>(tmax));
-        lazy_rescale<D / 16>(tmax, m, l, o);
-        // P = P_hi + P_lo, both bf16 (P_lo = the rounding error of P_hi): the
-        // two products keep P to ~2^-17 relative, where one bf16 P (2^-9)
-        // would be visible in bf16 outputs of few-key rows.
-        uint32_t ph[4], pl[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const float p0 = __builtin_amdgcn_exp2f(sc[2 * j] - m);
-            const float p1 = __builtin_amdgcn_exp2f(sc[2 * j + 1] - m);
-            l += p0 + p1;
-            ph[j] = pack_bf16x2(p0, p1);
-            pl[j] = pack_bf16x2(p0 - bf16_lo(ph[j]), p1 - bf16_hi(ph[j]));
-        }
-        const uint4 pop_hi = make_uint4(ph[0], ph[1], ph[2], ph[3]);
-        const uint4 pop_lo = make_uint4(pl[0], pl[1], pl[2], pl[3]);
-        // O^T += V^T P^T: A row i = d (16b + col), k = keys 8grp .. +7
-#pragma unroll
-        for (int b = 0; b < D / 16; ++b) {
-            const uint4 va = vop(b);
-            o[b] = mfma16(va, pop_lo, mfma16(va, pop_hi, o[b]));
-        }
-    };
-    // the padded, chunk-swizzled tile buffers of the register-staged paths
-    auto compute_tile = [&](int t0, auto buf_c) __attribute__((always_inline)) {
-        constexpr int BO = decltype(buf_c)::value * TILE;  // the tile's buffer
-        tile_core(
-            t0,
-            [&](int b, int c) __attribute__((always_inline)) {
-                // chunk grp + 4c of key row kr sits at (grp ^ s0) + 4 * (c ^ 2 s3)
-                // (s0, s3: bits 4 and 3 of kr): slices c with bit 1 clear read 64
-                // elements further when s3 is set, the others 64 nearer
-                const int kr = pf_key(b, col);
-                const int kd = D >= 128 ? ((kr >> 3) & 1) * 64 : 0;
-                const uint16_t *kp = &sk_w[BO + kr * KP + 8 * (grp ^ (D >= 128 ? (kr >> 4) & 1 : 0))];
-                return *reinterpret_cast<const uint4 *>(kp + 32 * c + ((c >> 1) & 1 ? -kd : kd));
-            },
-            [&](int b) __attribute__((always_inline)) {
-                return read_vt(((b >> 2) & 1 ? sv_hi : sv_lo) + BO + 16 * b);
-            });
-    };
-    // Q is in registers before the first prefetch is issued: inside the loop
-    // the compiler then waits only for each tile's own loads, not for the
-    // prefetches behind it (vmcnt counts in order).
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    if constexpr (RG) {
-        // LDS DMA ring: 32-key tile j (keys kstart + 32 j ..) goes to stage
-        // j % NS, K and V rows unpadded and chunk-swizzled (pf_rswz), by
-        // global_load_lds_dwordx4 (a 1 KiB row range per instruction, lane l
-        // fetching the logical chunk that lands on physical chunk l), the
-        // instructions of a tile spread over the waves. Groups of KS tiles
-        // are computed one after another (part p takes tile it * KS + p)
-        // while the next G - 1 groups are in flight; no registers hold them,
-        // and every wait is an explicit vmcnt on this wave's own DMAs (loads
-        // complete in issue order) followed by one barrier per group.
-        constexpr int RPI = 1024 / (2 * D);   // key rows per DMA instruction
-        constexpr int IPT = kPfKeys / RPI;    // instructions per K (or V) tile
-        constexpr int DPW = 2 * IPT / NW;     // instructions per wave and tile
-        static_assert((2 * IPT) % NW == 0, "a tile's DMAs split evenly over the waves");
-        const uint16_t *kg = static_cast<const uint16_t *>(a.kv.k);
-        const uint16_t *vg = static_cast<const uint16_t *>(a.kv.v);
-        const uint32_t sk_a = lds_addr(sk), sv_a = lds_addr(sv);
-        const int ntiles = kend > kstart ? (kend - kstart + kPfKeys - 1) / kPfKeys : 0;
-        const int ngroups = (ntiles + KS - 1) / KS;
-        const int lrow = lane / (D / 8), pchunk = lane % (D / 8);
-        auto issue_tile = [&](int j) __attribute__((always_inline)) {
-            const int t0 = kstart + j * kPfKeys;
-            const uint32_t stage = (uint32_t)((j % NS) * RSUB) * 2;
-#pragma unroll
-            for (int i = 0; i < DPW; ++i) {
-                const int q = wave + i * NW;      // < IPT: K instruction q, else V instruction q - IPT
-                const int ins = q % IPT;
-                const int r = ins * RPI + lrow;   // key row of this lane
-                const int64_t off = pf_row_offset<D, LAYOUT>(a.kv, slot, kvh, t0, kclamp, kend, r, bad);
-                const uint16_t *gp = (q < IPT ? kg : vg) + off + 8 * (pchunk ^ pf_rswz(r));
-                const uint32_t dst = (q < IPT ? sk_a : sv_a) + stage + (uint32_t)ins * 1024u;
-                dma_load16_cached(gp, __builtin_amdgcn_readfirstlane(dst));
-            }
-        };
-        int issued = min((G - 1) * KS, ntiles);
-        for (int j = 0; j < issued; ++j) issue_tile(j);
-        // this lane's rows and swizzles in a stage: S^T A operand of key
-        // pf_key(b, col) (logical chunk 4c + grp), V^T row 8grp + col/4 (+4)
-        // with logical chunk 2b + (col & 3) / 2 and half col & 1
-        const int kr0 = pf_key(0, col), kr1 = pf_key(1, col);
-        const int ksw0 = grp ^ pf_rswz(kr0), ksw1 = grp ^ pf_rswz(kr1);
-        const int rv = 8 * grp + (col >> 2);
-        const int vsw = ((col & 3) >> 1) ^ pf_rswz(rv);
-        const int voff = rv * D + 4 * (col & 1);
-        for (int it = 0; it < ngroups; ++it) {
-            // tiles issued after this group's: their DMAs may stay in flight
-            const int later = issued - min((it + 1) * KS, ntiles);
-            wait_vmem_steps<DPW, (G - 1) * KS>(later);
-            __syncthreads();  // every wave's DMAs of group it have landed; group it - 1 is done
-            const int next = min((it + G) * KS, ntiles);
-            for (int j = issued; j < next; ++j) issue_tile(j);  // into group it - 1's stages
-            issued = next;
-            const int j = it * KS + part;  // this wave's tile (wave-uniform)
-            const int tj = kstart + j * kPfKeys;
-            if (wlive && j < ntiles && (QB == 1 || (tj < wkend && tj + kPfKeys > wkstart))) {
-                const int sb = (j % NS) * RSUB;
-                tile_core(
-                    tj,
-                    [&](int b, int c) __attribute__((always_inline)) {
-                        const int kr = b ? kr1 : kr0, ksw = b ? ksw1 : ksw0;
-                        return *reinterpret_cast<const uint4 *>(&sk[sb + kr * D + 8 * ((4 * c) ^ ksw)]);
-                    },
-                    [&](int b) __attribute__((always_inline)) {
-                        typedef short v4s_t __attribute__((ext_vector_type(4)));
-                        const uint16_t *p = &sv[sb + voff + 8 * ((2 * b) ^ vsw)];
-                        const v4s_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                            (v4s_t __attribute__((address_space(3))) *)(p));
-                        const v4s_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                            (v4s_t __attribute__((address_space(3))) *)(p + 4 * D));
-                        const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
-                        return make_uint4(l2.x, l2.y, h2.x, h2.y);
-                    });
-            }
-        }
-    } else if constexpr (PF) {
-        // PD tiles in flight in registers (ring slot s holds tiles s, s + PD,
-        // ...; keys past kend read row kclamp: in bounds, never visible) and
-        // two tile buffers in LDS (tile i in buffer i % 2; PD is even). Per
-        // tile one barrier: after it, tile i is staged and every wave is done
-        // with tile i - 1, whose buffer then takes tile i + 1 while tile i is
-        // computed.
-        static_assert(PD % 2 == 0, "tile parity follows the ring slot");
-        u32x4_t kreg[PD][KU], vreg[PD][KU];
-        StaticFor<0, PD>::run([&](auto pc) {
-            constexpr int p = decltype(pc)::value;
-            pf_fetch<D, LAYOUT, TK, KU, 64 * NW>(a.kv, slot, kvh, kstart + p * TK, kclamp, kend, kreg[p], vreg[p], bad);
-        });
-        pf_stage<D, TK, KU, 64 * NW>(sk, sv, kreg[0], vreg[0]);
-        pf_fetch<D, LAYOUT, TK, KU, 64 * NW>(a.kv, slot, kvh, kstart + PD * TK, kclamp, kend, kreg[0], vreg[0], bad);
-        for (int t0 = kstart; t0 < kend; t0 += PD * TK) {
-            StaticFor<0, PD>::run([&](auto pc) {
-                constexpr int p = decltype(pc)::value;
-                constexpr int pn = (p + 1) % PD;  // ring slot of the next tile
-                const int tt = t0 + p * TK;
-                if (tt < kend) {
-                    __syncthreads();
-                    // Staged and refetched unconditionally (past kend the
-                    // rows are clamped reads, never computed): a conditional
-                    // load here leaves the compiler unsure which loads are
-                    // still in flight, and it then waits for all of them
-                    // (the next tiles' prefetches included) before staging.
-                    pf_stage<D, TK, KU, 64 * NW>(sk + (pn % 2) * TILE, sv + (pn % 2) * TILE, kreg[pn], vreg[pn]);
-                    pf_fetch<D, LAYOUT, TK, KU, 64 * NW>(a.kv, slot, kvh, tt + TK + PD * TK, kclamp, kend, kreg[pn],
-                                                         vreg[pn], bad);
-                    // this wave's 32 keys of the tile (wave-uniform)
-                    const int st = tt + part * kPfKeys;
-                    if (computes && st < kend) compute_tile(st, std::integral_constant<int, p % 2>{});
-                }
-            });
-        }
-    } else {
-        // D = 512 (no registers to spare for a prefetch ring): each key row of
-        // a tile is one LDS DMA of 64 x 16 B straight into the tile buffer
-        // (row pitch and chunk swizzle as pf_stage_unit: lane l fetches the
-        // logical chunk that lands on physical chunk l), issued by the waves in
-        // turn, one tile ahead, into the other buffer. Per tile: each wave
-        // waits for its own DMAs, then one barrier.
-        static_assert(D / 8 == 64, "one DMA instruction per key row");
-        const uint16_t *kg = static_cast<const uint16_t *>(a.kv.k);
-        const uint16_t *vg = static_cast<const uint16_t *>(a.kv.v);
-        const uint32_t sk_a = lds_addr(sk), sv_a = lds_addr(sv);
-        auto dma_tile = [&](int t0, int buf) __attribute__((always_inline)) {
-            for (int rr = wave; rr < 2 * kPfKeys; rr += NW) {  // rr < 32: K row rr, else V row rr - 32
-                const int kr = rr % kPfKeys;
-                const int64_t off = pf_row_offset<D, LAYOUT>(a.kv, slot, kvh, t0, kclamp, kend, kr, bad);
-                const uint16_t *g = (rr < kPfKeys ? kg : vg) + off + 8 * (lane ^ pf_swz<D>(kr));
-                const uint32_t dst = (rr < kPfKeys ? sk_a : sv_a) + (uint32_t)(buf * TILE + kr * KP) * 2;
-                dma_load16_cached(g, __builtin_amdgcn_readfirstlane(dst));
-            }
-        };
-        if (kstart < kend) dma_tile(kstart, 0);
-        for (int t0 = kstart; t0 < kend; t0 += 2 * kPfKeys) {
-            StaticFor<0, 2>::run([&](auto pc) {
-                constexpr int p = decltype(pc)::value;
-                const int tt = t0 + p * kPfKeys;
-                if (tt < kend) {
-                    wait_vmem<0>();  // this wave's rows of tile tt have landed
-                    __syncthreads();  // every wave's have; tile tt - 32's buffer is free
-                    if (tt + kPfKeys < kend) dma_tile(tt + kPfKeys, 1 - p);
-                    if (computes) compute_tile(tt, std::integral_constant<int, p>{});
-                }
-            });
-        }
-    }
-    if (bad) a.err[0] = 1;
-    l = pair<OpSum, 32>(pair<OpSum, 16>(l));
-    if constexpr (KS > 1) {
-        // Combine the key parts of each head in a fixed order: parts 1 ..
-        // KS - 1 leave (m, l) per query and their o in the drained tile
-        // buffers; part 0 rescales everything to the common max and adds.
-        __syncthreads();  // every wave is done with the tile buffers
-        // o as each lane holds it, [(part - 1) * hw + hidx][block b][lane]: the
-        // 64 lanes of a write or read touch 1 KiB of consecutive 16-B chunks (no
-        // bank conflicts; a [query][D] layout put the 16 queries of a half-wave
-        // D * 4 B apart, on the same banks)
-        float4 *xo = reinterpret_cast<float4 *>(sk);
-        float2 *xml = reinterpret_cast<float2 *>(sv);  // [((part - 1) * hw + hidx) * QB + qsub][16 queries]
-        if (computes && part > 0) {
-            const int e = ((part - 1) * hw + hidx) * QB + qsub;
-            float4 *dst = xo + (int64_t)e * (D / 16) * 64 + lane;
-#pragma unroll
-            for (int b = 0; b < D / 16; ++b) dst[64 * b] = make_float4(o[b][0], o[b][1], o[b][2], o[b][3]);
-            if (grp == 0) xml[e * 16 + col] = make_float2(m, l);
-        }
-        __syncthreads();
-        if (!computes || part > 0) return;
-        float M = m;
-#pragma unroll
-        for (int q = 1; q < KS; ++q) M = fmaxf(M, xml[(((q - 1) * hw + hidx) * QB + qsub) * 16 + col].x);
-        const float w0 = __builtin_amdgcn_exp2f(m - M);
-        l *= w0;
-#pragma unroll
-        for (int b = 0; b < D / 16; ++b) o[b] *= w0;
-#pragma unroll
-        for (int q = 1; q < KS; ++q) {
-            const int e = ((q - 1) * hw + hidx) * QB + qsub;
-            const float2 ml = xml[e * 16 + col];
-            const float w = __builtin_amdgcn_exp2f(ml.x - M);
-            l = fmaf(ml.y, w, l);
-            const float4 *src = xo + (int64_t)e * (D / 16) * 64 + lane;
-#pragma unroll
-            for (int b = 0; b < D / 16; ++b) {
-                const float4 x = src[64 * b];
-                o[b][0] = fmaf(x.x, w, o[b][0]);
-                o[b][1] = fmaf(x.y, w, o[b][1]);
-                o[b][2] = fmaf(x.z, w, o[b][2]);
-                o[b][3] = fmaf(x.w, w, o[b][3]);
-            }
-        }
-        m = M;
-    } else if (!computes) {
-        return;
-    }
-    if (!qvalid) return;
-    if (nks > 1) {  // this key range's partial: o unnormalised, (m, l)
-        const int64_t pi = (((int64_t)item * hq + head) * Qn + qr) * nks + ks;
-        float *po = a.part_o + pi * D + 4 * grp;
-#pragma unroll
-        for (int b = 0; b < D / 16; ++b)
-            *reinterpret_cast<float4 *>(po + 16 * b) = make_float4(o[b][0], o[b][1], o[b][2], o[b][3]);
-        if (grp == 0) a.part_ml[pi] = make_float2(m, l);
-        return;
-    }
-    const float inv = l > 0.f ? 1.0f / l : 0.f;
-    uint16_t *op = a.out + (((int64_t)item * hq + head) * Qn + qr) * D + 4 * grp;
-    // v_cvt_pk_bf16_f32: round to nearest even, as f32_to_bf16 for every
-    // non-NaN value, in one instruction per pair
-#pragma unroll
-    for (int b = 0; b < D / 16; ++b)
-        *reinterpret_cast<uint2 *>(op + 16 * b) =
-            make_uint2(pack_bf16x2(o[b][0] * inv, o[b][1] * inv), pack_bf16x2(o[b][2] * inv, o[b][3] * inv));
-}
-
-// Merge of a key-split prefill: one thread per (item, q head, query) row and
-// 4 consecutive dims (16-byte partial loads; D is a power of two, dshift =
-// log2(D / 4)), the n_ksplit partials in key order, bf16 out. Per dim the
-// arithmetic is merge_partials<1>'s (batches of 16 in partial order).
-__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a, int D, int dshift, int64_t outs4) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= outs4) return;
-    const int64_t row = t >> dshift;  // (item, q head, query)
-    const int d = (int)(t & ((1 << dshift) - 1)) * 4;
-    const int nks = a.n_ksplit;
-    const float2 *ml = a.part_ml + row * nks;
-    const float *po = a.part_o + row * nks * D + d;
-    constexpr int B = 16;
-    float M = kNegBig, L = 0.f;
-    float4 O = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int s0 = 0; s0 < nks; s0 += B) {
-        float2 m[B];
-        float4 v[B];
-#pragma unroll
-        for (int u = 0; u < B; ++u) {
-            const int sp = s0 + u;
-            m[u] = make_float2(kNegBig, 0.f);
-            v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (sp < nks) {
-                m[u] = ml[sp];
-                v[u] = *reinterpret_cast<const float4 *>(po + (int64_t)sp * D);
-            }
-        }
-        float bm = M;
-#pragma unroll
-        for (int u = 0; u < B; ++u) bm = fmaxf(bm, m[u].x);
-        const float c = __builtin_amdgcn_exp2f(M - bm);
-        L *= c;
-        O.x *= c;
-        O.y *= c;
-        O.z *= c;
-        O.w *= c;
-        M = bm;
-#pragma unroll
-        for (int u = 0; u < B; ++u) {
-            const float w = __builtin_amdgcn_exp2f(m[u].x - M);
-            L = fmaf(m[u].y, w, L);
-            O.x = fmaf(v[u].x, w, O.x);
-            O.y = fmaf(v[u].y, w, O.y);
-            O.z = fmaf(v[u].z, w, O.z);
-            O.w = fmaf(v[u].w, w, O.w);
-        }
-    }
-    const bool any = L > 0.f;
-    const uint2 packed = make_uint2(pack_bf16x2(any ? O.x / L : 0.f, any ? O.y / L : 0.f),
-                                    pack_bf16x2(any ? O.z / L : 0.f, any ? O.w / L : 0.f));
-    *reinterpret_cast<uint2 *>(a.out + row * D + d) = packed;
-}
-
-// ---------------------------------------------------------------------------
 // small control kernels
 // ---------------------------------------------------------------------------
 // One workgroup of kPtUpdates threads, thread i edits entry i.
@@ -3103,88 +2320,6 @@ hipError_t launch_decode_talker(const TalkerArgs &a, int head_dim, int rows_per_
         default: return hipErrorInvalidValue;
     }
     return hipErrorInvalidValue;
-}
-
-// The key-split merge: (item, q head, query) rows x D / 4 threads.
-hipError_t launch_prefill_merge(const PrefillArgs &a, int head_dim, hipStream_t s) {
-    if (head_dim < 4 || (head_dim & (head_dim - 1)) != 0) return hipErrorInvalidValue;
-    int dshift = 0;
-    while ((1 << dshift) < head_dim / 4) ++dshift;
-    const int64_t outs4 = (int64_t)a.n_items * a.kv.kv_heads * a.group * a.qn * (head_dim / 4);
-    hipLaunchKernelGGL(prefill_merge_kernel, dim3((unsigned)((outs4 + 255) / 256)), dim3(256), 0, s, a, head_dim,
-                       dshift, outs4);
-    return hipGetLastError();
-}
-
-hipError_t launch_prefill(const PrefillArgs &a, int head_dim, hipStream_t s) {
-    const int hw = a.heads_per_wg;
-    if (hw <= 0 || a.group % hw != 0 || hw > kPfMaxHeads) return hipErrorInvalidValue;
-    if (a.n_ksplit < 1 || (a.n_ksplit > 1 && (!a.part_o || !a.part_ml))) return hipErrorInvalidValue;
-    const int ks = a.key_parts;
-    if ((ks != 1 && ks != 2 && ks != 4) || ks > prefill_max_parts(head_dim) || hw * ks > 8) return hipErrorInvalidValue;
-    if (a.q_blocks != 1 && !(a.q_blocks == 2 && a.ring_groups)) return hipErrorInvalidValue;
-    if (a.kv.layout == KVRT_LAYOUT_RING && a.kv.rows < kPfKeys * ks) return hipErrorInvalidValue;  // one wrap per tile
-    if (a.ring_groups) {
-        // DMA ring: hw * ks * qb waves (at least 2), every one computing
-        const int g = a.ring_groups, qbk = a.q_blocks;
-        if (!prefill_ring_ok(head_dim, a.kv.layout, ks, g, qbk) || hw * ks * qbk > 8) return hipErrorInvalidValue;
-        dim3 grid(a.n_ksplit * a.kv.kv_heads * (a.group / hw), a.n_items, (a.qn + 16 * qbk - 1) / (16 * qbk));
-        const int nw = hw * ks * qbk < 2 ? 2 : hw * ks * qbk;
-        auto ring = [&](auto d_c, auto ks_c, auto qb_c) -> hipError_t {
-            constexpr int HD = decltype(d_c)::value, KS = decltype(ks_c)::value, QB = decltype(qb_c)::value;
-            constexpr int G = kPfRingGroups;
-            auto go = [&](auto nw_c) {
-                constexpr int NW = decltype(nw_c)::value;
-                if (a.kv.layout == KVRT_LAYOUT_RING)
-                    hipLaunchKernelGGL((prefill_kernel<HD, KVRT_LAYOUT_RING, NW, true, KS, G, QB>), grid,
-                                       dim3(64 * NW), 0, s, a);
-                else
-                    hipLaunchKernelGGL((prefill_kernel<HD, KVRT_LAYOUT_CONTIG, NW, true, KS, G, QB>), grid,
-                                       dim3(64 * NW), 0, s, a);
-            };
-            if (nw == 2) go(std::integral_constant<int, 2>{});
-            else if (nw == 4) go(std::integral_constant<int, 4>{});
-            else go(std::integral_constant<int, 8>{});
-            return hipGetLastError();
-        };
-        using C128 = std::integral_constant<int, 128>;
-        using C256 = std::integral_constant<int, 256>;
-        using I1 = std::integral_constant<int, 1>;
-        using I2 = std::integral_constant<int, 2>;
-        hipError_t e;
-        if (qbk == 2) e = ks == 1 ? ring(C128{}, I1{}, I2{}) : ring(C128{}, I2{}, I2{});
-        else if (head_dim == 256) e = ks == 1 ? ring(C256{}, I1{}, I1{}) : ring(C256{}, I2{}, I1{});
-        else e = ks == 1 ? ring(C128{}, I1{}, I1{}) : ring(C128{}, I2{}, I1{});
-        if (e != hipSuccess || a.n_ksplit == 1) return e;
-        return launch_prefill_merge(a, head_dim, s);
-    }
-    dim3 grid(a.n_ksplit * a.kv.kv_heads * (a.group / hw), a.n_items, (a.qn + 15) / 16);
-    // 4 or 8 waves (hw * ks compute); D = 512 keeps no tile in flight across
-    // the MFMAs (registers)
-    const bool w8 = hw * ks > 4;
-    auto go = [&](auto nw_c, auto ks_c) -> hipError_t {
-        constexpr int NW = decltype(nw_c)::value, KS = decltype(ks_c)::value;
-        KVRT_DISPATCH_D(head_dim, {
-            if constexpr (KS <= prefill_max_parts(HD)) {
-                KVRT_DISPATCH_LAYOUT(a.kv.layout, hipLaunchKernelGGL((prefill_kernel<HD, LY, NW, (HD < 512), KS>),
-                                                                     grid, dim3(64 * NW), 0, s, a));
-                return hipGetLastError();
-            } else {
-                return hipErrorInvalidValue;
-            }
-        });
-        return hipErrorInvalidValue;
-    };
-    using I1 = std::integral_constant<int, 1>;
-    using I2 = std::integral_constant<int, 2>;
-    using I4 = std::integral_constant<int, 4>;
-    using I8 = std::integral_constant<int, 8>;
-    hipError_t e;
-    if (ks == 1) e = w8 ? go(I8{}, I1{}) : go(I4{}, I1{});
-    else if (ks == 2) e = w8 ? go(I8{}, I2{}) : go(I4{}, I2{});
-    else e = w8 ? go(I8{}, I4{}) : go(I4{}, I4{});
-    if (e != hipSuccess || a.n_ksplit == 1) return e;
-    return launch_prefill_merge(a, head_dim, s);
 }
 
 hipError_t launch_set_lens(const SetLenArgs &a, hipStream_t s) {

@@ -2013,85 +2013,56 @@ int kvrt_attend_prefill_async(kvrt_ctx *c, int32_t layer, int32_t n, const int32
     a.group = group;
     a.qn = (int)qn;
     a.window = s.window;
-    // q heads per workgroup: the largest divisor of the group up to 8 at
-    // D 512 and up to 4 below (each further part of the group stages the K/V
-    // tiles again, but at D <= 256 twice the workgroups of 4 heads fill more
-    // of the chip: thinker sliding Q 291 44.0 -> 40.2 us, Q 2048 112.8 ->
-    // 107.1 us; at D 512 four heads per workgroup take 1.9x as long);
-    // KVRT_PF_HEADS_PER_WG lowers the cap
-    static const int hw_env = env_int("KVRT_PF_HEADS_PER_WG", kPfMaxHeads);
-    const int hw_cap = std::min(hw_env, D <= 256 ? 4 : kPfMaxHeads);
-    int hw = 1;
-    for (int d = 1; d <= std::min({group, kPfMaxHeads, hw_cap}); ++d)
-        if (group % d == 0) hw = d;
-    a.heads_per_wg = hw;
-    // Key parts: up to 8 waves per workgroup, hw heads x key_parts waves each
-    // splitting every tile's keys (the tile buffers bound the parts: 2 at
-    // D 256, 4 below, 1 at D 512; a ring needs a tile's keys to wrap at most
-    // once). More waves on each query block shorten the latency-bound chain
-    // of tiles of a short chunk: 2 parts took thinker sliding Q 291 from 36.9
-    // to 29.6 us, talker Q 512 from 33.6 to 29.7 us and thinker Q 2048 from
-    // 93.2 to 67.2 us; 4 parts (talker: 147 KB of LDS, one workgroup per CU)
-    // 43.9 us for the talker. KVRT_PF_KEY_PARTS caps it.
-    static const int parts_env = env_int("KVRT_PF_KEY_PARTS", 0);
-    const int64_t wgs_grid = (int64_t)((qn + 15) / 16) * hkv * (group / hw) * n;
-    int parts = std::min({parts_env > 0 ? parts_env : 2, prefill_max_parts(D), 8 / hw});
-    // a grid of two workgroups per CU needs no more waves per block (talker
-    // Q 512: 23.3 us with one part, 24.4 us with two); KVRT_PF_KEY_PARTS
-    // sets the parts there too
-    if (wgs_grid >= 512 && parts_env == 0) parts = 1;
-    parts = parts >= 4 ? 4 : parts >= 2 ? 2 : 1;
-    while (parts > 1 && s.layout == KVRT_LAYOUT_RING && s.ring_rows < kPfKeys * parts) parts /= 2;
-    a.key_parts = parts;
-    // LDS DMA ring (bf16 CONTIG / RING, D 128 / 256) instead of tiles staged
-    // through registers: KVRT_PF_RING = 1 / 0 forces it on / off
-    static const int ring_env = [] {
-        const char *e = std::getenv("KVRT_PF_RING");
-        return e && *e ? std::atoi(e) : -1;
-    }();
-    const bool ring_default = D == 128;
-    a.ring_groups = 0;
-    if ((ring_env > 0 || (ring_env < 0 && ring_default)) && prefill_ring_ok(D, s.layout, parts, kPfRingGroups) &&
-        (s.layout != KVRT_LAYOUT_RING || s.ring_rows >= kPfKeys))
-        a.ring_groups = kPfRingGroups;
-    // Talker-sized grids (>= 512 workgroups) on the ring at head_dim 128: two
-    // 16-query blocks per workgroup share its staged tiles, and with the LDS
-    // and waves this frees each block's keys go to two waves (talker Q 512:
-    // 22.1 -> 21.3 us; pairs with one key part were 2-5% faster than single
-    // blocks, four key parts without pairs took 40.0 us). KVRT_PF_QBLOCKS =
-    // 1 / 2 forces single blocks / pairs; KVRT_PF_KEY_PARTS sets the parts.
-    static const int qblocks_env = env_int("KVRT_PF_QBLOCKS", 0);
-    a.q_blocks = 1;
-    if (a.ring_groups && (qblocks_env == 2 || (qblocks_env == 0 && wgs_grid >= 512))) {
-        int p2 = parts_env > 0 ? parts : 2;
-        while (p2 > 1 && (hw * p2 * 2 > 8 || (s.layout == KVRT_LAYOUT_RING && s.ring_rows < kPfKeys * p2))) p2 /= 2;
-        if (hw * p2 * 2 <= 8 && prefill_ring_ok(D, s.layout, p2, a.ring_groups, 2)) {
-            a.q_blocks = 2;
-            parts = p2;
-            a.key_parts = parts;
-        }
-    }
-    // Key split: when the query blocks give fewer than 128 workgroups (a short
-    // chunk over a long context: thinker full layers, Q 291 over 2048 keys,
-    // 76 workgroups on 256 CUs), each block's keys are cut into n_ksplit
-    // ranges of >= 256 keys, as many as keep the grid within 256 workgroups
-    // (one round: a D 512 workgroup holds 135 KB of LDS, one per CU); a merge
-    // kernel then combines the ranges' partials. Q 291 at D 512: 213.8 us
-    // unsplit, 134.8 / 106.1 / 142.4 / 125.7 us with 2 / 3 / 4 / 6 ranges
-    // (4 ranges: 304 workgroups, a second round).
-    // Not inside a capture that would need a larger workspace.
-    // KVRT_PF_KSPLIT=1 turns it off, n >= 2 forces n ranges.
+    // Shape of the launch: row_waves 32-row blocks x key_parts per workgroup and
+    // key ranges per row block. A chunk's time is the chain of key blocks one
+    // wave walks (about 1.1 us a block at head_dim 256, 2 us at 512, 0.5 us
+    // below), so the smaller the grid, the more waves share a row block's keys,
+    // first inside a workgroup (combined through LDS), then over workgroups
+    // (partials in the workspace and a merge launch, ~6 us).
     static const int ksplit_env = env_int("KVRT_PF_KSPLIT", 0);
+    const int64_t rows = (int64_t)group * qn;
+    const auto wgs = [&](int w) { return (rows + 32 * w - 1) / (32 * w) * hkv * n; };  // workgroups of w row blocks
+    int rw = 4, parts = 1;
+    // least keys of a key range, and least keys that a split has to take off a
+    // workgroup's walk to be worth its merge (head_dim 512: one row block's
+    // accumulators fill the AGPRs and two staged groups the LDS: no parts)
+    int min_keys = 96, split_keys = 120;
+    if (D == 256) {
+        // a workgroup's 137 KB of LDS leave one per CU: past two rounds of
+        // them (without a window their lengths differ and the rounds overlap)
+        // four row blocks per workgroup and no parts are faster (window 512, 3
+        // streams x Q 1200: 44.6 -> 32.7 us; 4 x Q 600: 23.8 against 29.6 us);
+        // so are they where two parts would not have a block each
+        if (block_keys > 64 && wgs(2) <= (s.window > 0 ? 384 : 512)) rw = 2, parts = 2;
+        min_keys = 80, split_keys = 400;
+    } else if (D <= 128) {
+        // four parts while one round of workgroups takes the grid (Hq 16, one
+        // stream x Q 512: 10.0 us, two parts 12.2; x Q 800 over 2000: 35.1, 40.8),
+        // two up to two rounds of four row blocks (4 x Q 512: 15.4 us, four
+        // parts 20.4), none beyond (4 x Q 1400: 98.7 us, two parts 102.6). A
+        // PAGED row's address costs a lane more than its DMA: two row blocks
+        // share the fetching, and a split pays with half the keys.
+        if (wgs(1) <= 256 && s.layout != KVRT_LAYOUT_PAGED) rw = 1, parts = 4;
+        else if (wgs(2) < 256) rw = 2, parts = 4;
+        else if (wgs(4) < 512) rw = 2, parts = 2;
+        min_keys = s.layout == KVRT_LAYOUT_PAGED ? 180 : 360;
+        split_keys = s.layout == KVRT_LAYOUT_PAGED ? 250 : 500;
+    }
+    a.row_waves = rw;
+    a.key_parts = parts;
+    // Key ranges: as many as keep the grid within one round of 256 workgroups
+    // (Q 291 at head_dim 512 over 2339 keys, 4 streams: 156 us unsplit, 99 / 87 /
+    // 121 us with 2 / 3 / 4 ranges). Not inside a capture that would need a
+    // larger workspace. KVRT_PF_KSPLIT=1 turns it off, n >= 2 forces n ranges.
     a.n_ksplit = 1;
-    const int64_t wgs1 = (int64_t)((qn + 15) / 16) * hkv * (group / hw) * n;
-    if (ksplit_env != 1 && (ksplit_env > 1 || wgs1 < 128) && block_keys >= 512) {
-        const int64_t want = ksplit_env > 1 ? ksplit_env : std::min<int64_t>(256 / wgs1, block_keys / 256);
-        const int nks = (int)std::max<int64_t>(1, std::min<int64_t>(want, 16));
+    const int64_t want = ksplit_env > 0 ? ksplit_env : std::min<int64_t>(256 / wgs(rw), block_keys / min_keys);
+    const int nks = (int)std::min<int64_t>(want, 16);
+    if (nks > 1 && (ksplit_env > 0 || block_keys * (nks - 1) / nks >= split_keys)) {
         const size_t po = ((size_t)n * hq * qn * nks * D + 63) / 64 * 64;
         const size_t bytes = po * 4 + (size_t)n * hq * qn * nks * 8 + 256;
         hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
         const bool capturing = hipStreamIsCapturing(c->stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
-        if (nks > 1 && (bytes <= c->ws_bytes || (!capturing && ensure_workspace(c, bytes) == KVRT_OK))) {
+        if (bytes <= c->ws_bytes || (!capturing && ensure_workspace(c, bytes) == KVRT_OK)) {
             a.n_ksplit = nks;
             a.part_o = c->ws;
             a.part_ml = reinterpret_cast<float2 *>(c->ws + po);

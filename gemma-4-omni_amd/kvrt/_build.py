@@ -1,7 +1,8 @@
 """Build libkvrt.so (gfx950) in-tree with hipcc.
 
-The library is compiled from ``csrc/kvrt_kernels.hip`` (kernels) and
-``csrc/kvrt_runtime.hip`` (host runtime, C ABI in ``include/kvrt.h``). The
+The library is compiled from ``csrc/kvrt_kernels.hip`` (kernels),
+``csrc/kvrt_prefill.hip`` (chunked prefill) and ``csrc/kvrt_runtime.hip`` (host
+runtime, C ABI in ``include/kvrt.h``). The
 build also compiles ``csrc/kvrt_coherence_probe.hip`` to assembly (never
 linked) and fails if the coherent-access helpers lower differently from what
 the single-launch decode merge relies on.
@@ -21,7 +22,9 @@ PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR.parent / "csrc"
 INCLUDE = PKG_DIR.parent.parent / "include"
 LIB_PATH = PKG_DIR / "libkvrt.so"
-SOURCES = ("kvrt_kernels.hip", "kvrt_runtime.hip")
+SOURCES = ("kvrt_kernels.hip", "kvrt_prefill.hip", "kvrt_prefill_wide.hip", "kvrt_runtime.hip")
+
+AGPR_SOURCES = ("kvrt_prefill_wide.hip",)
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -31,18 +34,21 @@ HIPCC_FLAGS = [
     # Packed FP32 VALU forms are kept out of every code object.
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-fhip-fp32-correctly-rounded-divide-sqrt",
-    # MFMA accumulators live in ordinary VGPRs. With the default AGPR form the
+    # (all sources but the wide prefill's:) MFMA accumulators live in ordinary VGPRs. With the default AGPR form the
     # prefill tile loop copied its output accumulators between the two
     # register files every tile (72 v_accvgpr moves per 32-key tile at D 128);
     # the VGPR form drops them and raises occupancy of several decode and
     # prefill instantiations (talker prefill 26.4 -> 23.8 us per launch).
-    "-mllvm", "-amdgpu-mfma-vgpr-form=1",
     "-Wall",
     "-Wno-unused-function",
     # flowing off the end of a value-returning function is undefined (a
     # launcher lambda that did so crashed the host): refuse to build it
     "-Werror=return-type",
 ]
+
+
+def mfma_flags(source: str) -> list[str]:
+    return [] if source in AGPR_SOURCES else ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
 
 
 def hipcc() -> str:
@@ -72,7 +78,7 @@ def _resources(stderr: str) -> dict[str, dict[str, str]]:
 
 
 def _compile(src: Path, obj: Path) -> dict[str, dict[str, str]]:
-    cmd = [hipcc(), *HIPCC_FLAGS, f"-I{INCLUDE}", "-c", str(src), "-o", str(obj),
+    cmd = [hipcc(), *HIPCC_FLAGS, *mfma_flags(src.name), f"-I{INCLUDE}", "-c", str(src), "-o", str(obj),
            "-Rpass-analysis=kernel-resource-usage"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:

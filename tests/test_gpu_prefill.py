@@ -102,6 +102,53 @@ def test_prefill_matches_oracle(hq, hkv, d, window, layout, prefix, qn):
     _check(rt, orc, q, 1.0 / math.sqrt(d))
 
 
+@pytest.mark.parametrize("d", [64, 128, 256, 512])
+@pytest.mark.parametrize(
+    "hq,hkv,window,layout,prefix,qn,scale,grow",
+    [
+        # last row of a 32-row block, one past it, one short of it
+        (8, 1, 0, "contig", [0], 4, 1.0, 0.0),
+        (8, 1, 0, "contig", [29, 31, 32, 33], 5, 1.0, 0.0),
+        (5, 1, 0, "contig", [64], 13, 1.0, 0.0),
+        (1, 1, 0, "contig", [0, 95], 33, 1.0, 0.0),
+        # more row blocks than one workgroup's, keys split over workgroups
+        (12, 2, 0, "contig", [1100, 3], 23, 1.0, 0.0),
+        (8, 1, 90, "ring", [700, 40], 37, 1.0, 0.0),
+        (8, 2, 0, "paged", [513], 31, 1.0, 0.0),
+        # scores that rise along the keys move the running max again and again
+        (8, 1, 0, "contig", [600], 9, 1.0, 12.0),
+        (8, 1, 0, "contig", [300], 20, -1.0, 12.0),
+        (8, 1, 200, "ring", [90], 64, 0.0, 0.0),
+    ],
+)
+def test_prefill_row_blocks_and_key_blocks_at_their_edges(d, hq, hkv, window, layout, prefix, qn, scale, grow):
+    """Rows (q heads x queries) in blocks of 32, keys in blocks of 32 over 1, 2
+    or 4 parts and over workgroups; scales of either sign and zero. With
+    ``grow`` the keys' lengths rise along the positions (scores of up to about
+    grow * 8 log2 units), so that the accumulators are rescaled; outputs are
+    then single values of N(0,1) rather than averages. Bound: an output's
+    rounding to bf16 is at most 2^-8 of it, and 2e-3 covers the rest: |v| < 5
+    times the weights' error, 2^-17 from their two bf16 terms and 100 * 2^-20
+    from scores of up to 100 summed and scaled in fp32."""
+    rt, orc, q = _setup(hq, hkv, d, window, layout, prefix, qn, seed=d + hq + qn)
+    if grow:
+        L = prefix[0] + qn
+        k, v, _, _ = rt.storage(0)
+        ramp = torch.linspace(0.05, grow, L).to(torch.bfloat16).float()
+        kk = (k[0, :, :L].float().cpu() * ramp[None, :, None]).to(torch.bfloat16)
+        vv = v[0, :, :L].clone()
+        k[0, :, :L] = kk.cuda()
+        orc = O.OracleCache([O.OracleLayer(hkv, d, window)], 1)
+        orc.append(0, 0, to_np(kk), to_np(vv))
+        q = q * 2
+    n = q.shape[0]
+    out = rt.attend_prefill(0, q.cuda(), list(range(n)), scale / math.sqrt(d))
+    assert rt.health() == 0
+    for i in range(n):
+        ref = orc.attend(i, 0, to_np(q[i]), scale / math.sqrt(d))
+        assert (np.abs(to_np(out[i]) - ref) <= 2.0 ** -8 * np.abs(ref) + 2e-3).all()
+
+
 def test_prefill_single_query_and_decode_dispatch():
     """Q = 1 through the MFMA kernel; g * Q above 16 rows dispatches to it from attend()."""
     rt, orc, q = _setup(2, 1, 128, 0, "contig", [77], 1, seed=5)

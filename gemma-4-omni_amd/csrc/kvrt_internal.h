@@ -353,6 +353,27 @@ struct SlotMoveArgs {
     int32_t rows[kMaxMoveLayers];
 };
 
+// Opening of a session in one slot: every stored row of the CONTIG and RING
+// layers listed (bf16) is written once, from the imported K / V where a
+// position of [0, rows) lives in it and as zeros elsewhere; their device
+// lengths become rows and the slot's prefix mask is cleared.
+constexpr int kMaxOpenLayers = 48;  // layers per launch (2.7 KB of arguments)
+struct OpenLayer {
+    const uint16_t *k;        // [kv_heads, rows, D], rows head_stride / row_stride elements apart
+    const uint16_t *v;
+    int64_t head_stride, row_stride;
+    int32_t layer;
+    int32_t rows;             // 0: the layer is emptied
+};
+struct OpenArgs {
+    const LayerDesc *desc;
+    int32_t *lens;            // [slots, layers]
+    int32_t *prefix_len;      // of the slot
+    int32_t slot;
+    int32_t n_layers;
+    OpenLayer l[kMaxOpenLayers];
+};
+
 struct CopyRowsArgs {
     const uint8_t *src;
     uint8_t *dst;
@@ -385,6 +406,8 @@ hipError_t launch_slot_copy(const SlotMoveArgs &a, int64_t max_units, hipStream_
 // In-place move of <= kMaxRebaseRows rows per entry within one slot, keys
 // rotated by rope_delta positions where the layer has a RoPE table (bf16).
 hipError_t launch_slot_rebase(const SlotMoveArgs &a, int max_heads, hipStream_t s);
+// n entries; max_heads and max_units (16-B units of a head's rows) over them.
+hipError_t launch_open_slot(const OpenArgs &a, int n, int max_heads, int64_t max_units, hipStream_t s);
 hipError_t launch_zero(void *p, uint64_t bytes, hipStream_t s);
 hipError_t launch_prefix_pack(const PrefixPackArgs &a, hipStream_t s);
 

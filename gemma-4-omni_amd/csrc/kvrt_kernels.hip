@@ -9,6 +9,7 @@
 //   merge_kernel    log-sum-exp merge of the partials in fixed order
 //                   (deterministic) -> bf16, then the fused length advance
 //   set_i32_kernel  length / page-table edits carried in the kernarg block
+//   open_slot_kernel  a session's rows imported (or zeroed) over all layers of a slot
 //   copy_rows_kernel, zero_kernel, slot_copy_kernel, slot_rebase_kernel
 //
 // Every memory-bound loop moves 16 B per lane with consecutive lanes on
@@ -2132,6 +2133,47 @@ __global__ __launch_bounds__(512) void prefix_pack_kernel(PrefixPackArgs a) {
     if (t == 0) m->len = a.plen;
 }
 
+// Grid (row chunks, heads, 2 * layers): block (x, y, 2e + j) writes kOpenUnits
+// 16-B units per thread of head y of layer e's K (j = 0) or V rows. One pass
+// over the slot instead of a fill and a copy per layer and tensor, HBM-bound:
+// 28 layers of 8 heads x 1024 rows x 128, 700 of them imported, took 57 fills
+// (2.2 us each) and 28 copies (4.3 us), now one launch of 46 us (198 MB).
+constexpr int kOpenUnits = 4;
+__global__ __launch_bounds__(256) void open_slot_kernel(OpenArgs a) {
+    const OpenLayer &L = a.l[blockIdx.z >> 1];
+    const bool is_v = blockIdx.z & 1;
+    const LayerDesc &T = a.desc[L.layer];
+    const int head = blockIdx.y;
+    if (blockIdx.x == 0 && head == 0 && !is_v && threadIdx.x == 0) {
+        a.lens[(int64_t)a.slot * a.n_layers + L.layer] = L.rows;
+        if (blockIdx.z == 0) *a.prefix_len = 0;
+    }
+    if (head >= T.kv.kv_heads) return;
+    const int D = T.head_dim, ushift = __builtin_ctz((unsigned)D) - 3;  // D / 8 units per row, a power of two
+    const int stored = T.kv.rows, rows = L.rows;
+    // row r holds position r, or in a ring that has wrapped the one of
+    // [rows - stored, rows) that lives there
+    const int base = max(0, rows - stored), first = base % stored;
+    uint16_t *dst = static_cast<uint16_t *>(is_v ? T.kv.v : T.kv.k) + a.slot * T.kv.slot_stride + head * T.kv.head_stride;
+    const uint16_t *src = (is_v ? L.v : L.k) + head * L.head_stride;
+    const int64_t u0 = (int64_t)blockIdx.x * (256 * kOpenUnits) + threadIdx.x, units = (int64_t)stored << ushift;
+    uint4 x[kOpenUnits];
+#pragma unroll
+    for (int i = 0; i < kOpenUnits; ++i) {
+        const int64_t u = u0 + 256 * i;
+        const int r = (int)(u >> ushift);
+        const int pos = base + (r >= first ? r - first : r - first + stored);
+        x[i] = make_uint4(0, 0, 0, 0);
+        if (u < units && pos < rows)
+            x[i] = load_stream16(src + pos * L.row_stride + 8 * (u & ((1 << ushift) - 1)));
+    }
+#pragma unroll
+    for (int i = 0; i < kOpenUnits; ++i) {
+        const int64_t u = u0 + 256 * i;
+        if (u < units) *reinterpret_cast<uint4 *>(dst + 8 * u) = x[i];
+    }
+}
+
 __global__ __launch_bounds__(256) void zero_kernel(uint4 *p, uint64_t n16) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n16;
          i += (uint64_t)gridDim.x * blockDim.x)
@@ -2374,6 +2416,13 @@ hipError_t launch_prefix_pack(const PrefixPackArgs &a, hipStream_t s) {
     if (a.n_items <= 0) return hipSuccess;
     if (a.n_items > kMaxItems || a.plen < 0 || a.plen > KVRT_MAX_PREFIX_MASK) return hipErrorInvalidValue;
     hipLaunchKernelGGL(prefix_pack_kernel, dim3(a.n_items), dim3(512), 0, s, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_open_slot(const OpenArgs &a, int n, int max_heads, int64_t max_units, hipStream_t s) {
+    if (n <= 0 || n > kMaxOpenLayers || max_heads <= 0 || max_units <= 0) return hipErrorInvalidValue;
+    const int64_t gx = (max_units + 256 * kOpenUnits - 1) / (256 * kOpenUnits);
+    hipLaunchKernelGGL(open_slot_kernel, dim3((unsigned)gx, max_heads, 2 * n), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

@@ -1409,27 +1409,57 @@ int kvrt_write_positions_async(kvrt_ctx *c, int32_t layer, int32_t n, const int3
     return KVRT_OK;
 }
 
-int kvrt_reset_slot_async(kvrt_ctx *c, int32_t slot) {
-    int rc = begin(c);
-    if (rc) return rc;
-    if (!valid_slot(c, slot)) return KVRT_EINVAL;
+// Empties a slot and writes the given layers' imports (k, v null: none) into it,
+// all CONTIG and RING layers in one launch. The caller has checked everything.
+static int open_slot(kvrt_ctx *c, int32_t slot, int32_t n, const kvrt_tensor *k, const kvrt_tensor *v) {
+    OpenArgs a{};
+    a.desc = c->d_desc;
+    a.lens = c->d_len;
+    a.prefix_len = reinterpret_cast<int32_t *>(c->d_prefix + slot);
+    a.slot = slot;
+    a.n_layers = c->cfg.n_layers;
+    int entries = 0, heads = 0;
+    int64_t units = 0;
+    bool opened = false;
+    auto flush = [&]() -> int {
+        if (entries == 0) return KVRT_OK;
+        c->counters.launches++;
+        if (launch_open_slot(a, entries, heads, units, enq(c)) != hipSuccess) return poison(c);
+        entries = heads = 0;
+        units = 0;
+        opened = true;
+        return KVRT_OK;
+    };
     std::vector<int32_t> idx;
+    int rc = KVRT_OK;
     for (int l = 0; l < c->cfg.n_layers; ++l) {
         if (c->layers[l].owner != l) continue;
         const kvrt_layer_spec &s = c->layers[l].spec;
-        if (s.layout != KVRT_LAYOUT_PAGED) {
-            const KVView vw = make_view(c, l);
-            const uint64_t bytes = (uint64_t)vw.slot_stride * 2;
-            for (void *base : {vw.k, vw.v}) {
-                c->counters.launches++;
-                if (launch_zero(static_cast<uint8_t *>(base) + (uint64_t)slot * bytes, bytes, enq(c)) != hipSuccess)
-                    return poison(c);
+        const int S = k && l < n ? (int)k[l].dims[2] : 0;
+        if (s.layout == KVRT_LAYOUT_PAGED) {
+            idx.push_back((int32_t)((size_t)slot * c->cfg.n_layers + l));
+        } else {
+            OpenLayer &e = a.l[entries++];
+            e = OpenLayer{};
+            e.layer = l;
+            e.rows = S;
+            if (S > 0) {
+                e.k = static_cast<const uint16_t *>(k[l].data);
+                e.v = static_cast<const uint16_t *>(v[l].data);
+                e.head_stride = k[l].strides[1];
+                e.row_stride = k[l].strides[2];
             }
+            const KVView vw = make_view(c, l);
+            heads = std::max(heads, (int)s.kv_heads);
+            units = std::max(units, vw.head_stride / 8);
+            if (entries == kMaxOpenLayers && (rc = flush()) != KVRT_OK) return rc;
         }
-        c->len_ref(slot, l) = 0;
-        c->ring_set(slot, l, 0);
-        idx.push_back((int32_t)((size_t)slot * c->cfg.n_layers + l));
+        c->len_ref(slot, l) = S;
+        c->ring_set(slot, l, s.layout == KVRT_LAYOUT_RING ? std::max(0, S - s.ring_rows) : 0);
+        c->counters.appended_rows += (uint64_t)S * s.kv_heads;
+        c->counters.appended_bytes += (uint64_t)S * s.kv_heads * s.head_dim * 2 * 2;
     }
+    if ((rc = flush()) != KVRT_OK) return rc;
     if (c->paged) {
         for (int p = 0; p < c->pt_stride; ++p) {
             int32_t &e = c->pt[(size_t)slot * c->pt_stride + p];
@@ -1441,11 +1471,65 @@ int kvrt_reset_slot_async(kvrt_ctx *c, int32_t slot) {
         }
         c->first_live[slot] = 0;
     }
-    rc = set_device_lens(c, idx);
-    if (rc != KVRT_OK) return rc;
-    rc = set_prefix_len_device(c, slot, 0);
-    if (rc != KVRT_OK) return rc;
+    if ((rc = set_device_lens(c, idx)) != KVRT_OK) return rc;
+    if (!opened && (rc = set_prefix_len_device(c, slot, 0)) != KVRT_OK) return rc;
+    c->slot[slot].prefix_len = 0;
     renew_generation(c, slot);
+    return KVRT_OK;
+}
+
+int kvrt_reset_slot_async(kvrt_ctx *c, int32_t slot) {
+    int rc = begin(c);
+    if (rc) return rc;
+    if (!valid_slot(c, slot)) return KVRT_EINVAL;
+    return open_slot(c, slot, 0, nullptr, nullptr);
+}
+
+int kvrt_open_session_async(kvrt_ctx *c, int32_t slot, int32_t n, const kvrt_tensor *k, const kvrt_tensor *v) {
+    int rc = begin(c);
+    if (rc) return rc;
+    if (!valid_slot(c, slot) || n < 0 || (n > 0 && (!k || !v))) return KVRT_EINVAL;
+    // One launch where every import would be accepted and reads nothing of the
+    // slot itself; else the reset and the imports one by one, which refuse
+    // where they always did.
+    bool one = !c->lens_stale && n <= c->cfg.n_layers;
+    int imports = 0;
+    for (int l = 0; one && l < n; ++l) {
+        if (c->layers[l].owner != l) continue;
+        const kvrt_layer_spec &s = c->layers[l].spec;
+        one = s.layout != KVRT_LAYOUT_PAGED && tensor_ok_or_empty(&k[l], KVRT_BF16, 4) &&
+              tensor_ok_or_empty(&v[l], KVRT_BF16, 4);
+        for (int i = 0; one && i < 4; ++i)
+            one = k[l].dims[i] == v[l].dims[i] && (k[l].dims[2] == 0 || k[l].strides[i] == v[l].strides[i]);
+        one = one && k[l].dims[0] == 1 && k[l].dims[1] == s.kv_heads && k[l].dims[3] == s.head_dim &&
+              k[l].dims[2] >= 0 && k[l].dims[2] <= c->cfg.capacity;
+        ++imports;
+    }
+    auto reads_slot = [&](const kvrt_tensor &t) {
+        const char *lo = static_cast<const char *>(t.data);
+        const char *hi = lo + ((t.dims[1] - 1) * t.strides[1] + (t.dims[2] - 1) * t.strides[2] + t.dims[3]) * 2;
+        for (int m = 0; m < c->cfg.n_layers; ++m) {
+            if (c->layers[m].owner != m || c->layers[m].spec.layout == KVRT_LAYOUT_PAGED) continue;
+            const KVView w = make_view(c, m);
+            for (const void *base : {w.k, w.v}) {
+                const char *b = static_cast<const char *>(base) + (int64_t)slot * w.slot_stride * 2;
+                if (lo < b + w.slot_stride * 2 && b < hi) return true;
+            }
+        }
+        return false;
+    };
+    for (int l = 0; one && l < n; ++l)
+        if (c->layers[l].owner == l && k[l].dims[2] > 0) one = !reads_slot(k[l]) && !reads_slot(v[l]);
+    if (one) {
+        if ((rc = open_slot(c, slot, n, k, v)) != KVRT_OK) return rc;
+        for (int i = 0; i < imports; ++i) renew_generation(c, slot);  // as the imports do
+        return KVRT_OK;
+    }
+    if ((rc = kvrt_reset_slot_async(c, slot)) != KVRT_OK) return rc;
+    for (int l = 0; l < n; ++l) {
+        if (l < c->cfg.n_layers && c->layers[l].owner != l) continue;
+        if ((rc = kvrt_import_async(c, slot, l, &k[l], &v[l], 0)) != KVRT_OK) return rc;
+    }
     return KVRT_OK;
 }
 

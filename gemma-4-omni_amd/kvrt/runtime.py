@@ -13,6 +13,7 @@ from __future__ import annotations
 
 import ctypes
 import math
+import struct
 import threading
 from dataclasses import dataclass
 from typing import Iterable, Sequence
@@ -75,6 +76,9 @@ def tensor_desc(t: torch.Tensor) -> L.KvrtTensor:
     _DESC_CACHE[key] = d
     return d
 
+
+_DESC = struct.Struct("@Pii4q4q")  # one kvrt_tensor
+assert _DESC.size == ctypes.sizeof(L.KvrtTensor) and L.KVRT_MAX_RANK == 4
 
 _RAW_STREAM = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
@@ -443,6 +447,22 @@ class KVRuntime:
         # the mask is read on the stream: keep it alive until that work has run
         mask.record_stream(torch.cuda.current_stream(self.device))
 
+    def _session_descs(self, layers: Sequence[tuple[torch.Tensor, torch.Tensor]]) -> tuple[bytes, bytes] | None:
+        """The layers' K and V descriptors as two packed kvrt_tensor arrays; None
+        unless every one is a 4-D GPU tensor of a dtype a descriptor can name."""
+        if len(layers) > len(self.layers):
+            return None
+        k_all, v_all = [], []
+        for i, kv in enumerate(layers):
+            for t, out in ((kv[0], k_all), (kv[1], v_all)) if self._owner(i) == i else ():
+                if not t.is_cuda or t.dim() != 4 or t.dtype not in _DTYPE_CODES:
+                    return None
+                out.append(_DESC.pack(t.data_ptr(), _DTYPE_CODES[t.dtype], 4, *t.shape, *t.stride()))
+            if len(k_all) == i:  # a shared layer's entries are not read
+                k_all.append(bytes(_DESC.size))
+                v_all.append(bytes(_DESC.size))
+        return b"".join(k_all), b"".join(v_all)
+
     def import_session(self, slot: int, layers: Sequence[tuple[torch.Tensor, torch.Tensor]],
                        prefix_attention: torch.Tensor | None = None) -> int:
         """Start a session in ``slot``: reset it, import one HF layer view
@@ -450,11 +470,17 @@ class KVRuntime:
         shared layers' entries are ignored) and set its prefix mask. Returns
         the slot's generation. Mirrors gemma4_listener_batch_import_cache_async
         (gemma4_listener_microbatch_impl.inc:2590-2640)."""
-        self.reset_slot(slot)
-        for i, kv in enumerate(layers):
-            if self._owner(i) != i:
-                continue
-            self.import_(slot, i, kv[0], kv[1])
+        descs = self._session_descs(layers)
+        if descs is not None:
+            self._bind()
+            _check(self.lib.kvrt_open_session_async(self._ctx, int(slot), len(layers), *descs),
+                   "kvrt_open_session_async")
+        else:  # the single calls raise where a tensor is not one they take
+            self.reset_slot(slot)
+            for i, kv in enumerate(layers):
+                if self._owner(i) != i:
+                    continue
+                self.import_(slot, i, kv[0], kv[1])
         if prefix_attention is not None:
             self.set_prefix_attention(slot, prefix_attention)
         return self.slot_generation(slot)

@@ -8,8 +8,8 @@ native KV storage. These helpers take an HF ``DynamicCache`` into a
 * ``dynamic_cache_kv_layers`` — validate and borrow the exact bf16 layer
   tensors of an HF cache without casting or cloning
   (duplex_kernel/native_qwen_talker.py:350-392);
-* ``import_dynamic_cache`` — reset the slot, then one kvrt import launch per
-  layer (native_qwen_talker.py:781-874 -> qwen_talker.cu:1060-1110: memset
+* ``import_dynamic_cache`` — reset the slot and import every layer in one
+  launch (native_qwen_talker.py:781-874 -> qwen_talker.cu:1060-1110: memset
   of the arena, then the prefix copy);
 * ``advance_audio_q1_position`` — next causal Q1 position, failing closed
   past the response budget (native_qwen_talker.py:395-401).
@@ -80,10 +80,8 @@ def import_dynamic_cache(cache: Any, target: KVRTCache) -> int:
     for i, (k, v) in enumerate(layers):
         if not k.is_cuda:
             raise ValueError(f"DynamicCache layer {i} is not on the GPU (kvrt has no CPU path)")
-    target.reset()
-    for i, (k, v) in enumerate(layers):
-        if rt._owner(i) == i:
-            rt.import_(target.slot, i, k, v)
+    target.shared_layers.clear()
+    rt.import_session(target.slot, layers)
     target.adopt()
     return seq
 

@@ -263,6 +263,16 @@ int kvrt_layer_storage(kvrt_ctx *ctx, int32_t layer, kvrt_storage *out);
 int kvrt_import_async(kvrt_ctx *ctx, int32_t slot, int32_t layer, const kvrt_tensor *k,
                       const kvrt_tensor *v, int32_t first_pos);
 
+/* Start a session in a slot: kvrt_reset_slot_async, then kvrt_import_async of
+ * k[l], v[l] (first_pos 0) for every layer l < n that owns its storage (a
+ * shared layer's entries are not read). Where all of them are accepted and the
+ * layers are CONTIG or RING this is one launch that writes every stored row
+ * once; the results, refusals and generations are those of the single calls.
+ * k, v: arrays of n descriptors. Mirrors
+ * gemma4_listener_batch_import_cache_async (gemma4_listener_microbatch_impl.inc:2590-2640). */
+int kvrt_open_session_async(kvrt_ctx *ctx, int32_t slot, int32_t n, const kvrt_tensor *k,
+                            const kvrt_tensor *v);
+
 /* Append Q rows to n slots of one layer at each slot's current length:
  * k, v are [n, kv_heads, Q, D] bf16 (HF key_states layout with batch = n).
  * Lengths advance by Q. INT8 layers quantise in-kernel

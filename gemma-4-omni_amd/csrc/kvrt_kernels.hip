@@ -1087,8 +1087,9 @@ __device__ __forceinline__ void lazy_rescale(float tmax, float &m, float &l, f32
 }
 
 // Split-K decode on MFMA for R = g*Q in {8, 16} query rows per kv head
-// (bf16): same grid, key splits, visibility and partial format as
-// decode_kernel, one partial per workgroup. Per 16-key tile a wave computes
+// (bf16): same grid, visibility and partial format as decode_kernel, one
+// partial per workgroup, keys dealt in whole tiles (wave_tiles). Per 16-key
+// tile a wave computes
 //   S^T (16 keys x 16 rows) = K Q^T   D/32 v_mfma_f32_16x16x32_bf16, K read
 //                                     straight from HBM as the A operand
 //   O^T (D x 16) += V^T P^T           2 * D/16 v_mfma_f32_16x16x16_bf16
@@ -1182,6 +1183,21 @@ __device__ __forceinline__ void mfma_decode_finish(const DecodeArgs &a, uint8_t 
     if (a.cnt) decode_merge_tail<D, R>(a, item, kvh, hkv, rows);
 }
 
+// Keys [ws, we) of one wave of a bf16 MFMA decode: the item's tiles of T keys
+// are dealt as evenly as they go, contiguous per wave, the waves numbered
+// across the workgroups first so that the tiles left over fall on different
+// ones. (Every wave rounded up to whole tiles left up to a fifth of the
+// workgroups without keys while the rest read theirs: D 512 x 8300 keys, 1
+// stream 21.3 -> 18.8 us, 4 streams 24.8 -> 22.8; D 256 x 16500 15.7 -> 14.7.)
+template <int T>
+__device__ __forceinline__ void wave_tiles(int kstart, int kend, int wave, int &ws, int &we) {
+    const int n = gridDim.x * kWaves, rank = wave * gridDim.x + blockIdx.x;
+    const int tiles = (max(0, kend - kstart) + T - 1) / T;
+    const int base = tiles / n, rem = tiles - base * n;
+    ws = kstart + T * (rank * base + min(rank, rem));
+    we = min(kend, ws + T * (base + (rank < rem ? 1 : 0)));
+}
+
 template <int D, int R, int LAYOUT, int KDT = KVRT_BF16>
 __global__ __launch_bounds__(256) void decode_mfma_kernel(DecodeArgs a) {
     constexpr int T = kMfmaDecodeKeys;
@@ -1216,7 +1232,6 @@ __global__ __launch_bounds__(256) void decode_mfma_kernel(DecodeArgs a) {
     const int col = lane & 15, grp = lane >> 4;
     const int item = LAYOUT == KVRT_LAYOUT_PAGED ? launch_item(a, blockIdx.z) : (int)blockIdx.z;
     const int kvh = blockIdx.y, hkv = gridDim.y;
-    const int split = blockIdx.x * kWaves + wave;
     const int slot = a.slots[item];
     // The scalar arguments of the set-up, loaded in one batch with the slot
     // (one round trip) rather than each at its first use
@@ -1242,11 +1257,8 @@ __global__ __launch_bounds__(256) void decode_mfma_kernel(DecodeArgs a) {
     }
     const int p0 = kend - Qn;
     const int kstart = a.window > 0 ? max(0, p0 - a.window + 1) : 0;
-    const int nk = max(0, kend - kstart);
-    int chunk = (nk + a.n_split - 1) / a.n_split;
-    chunk = (chunk + T - 1) / T * T;
-    const int ws = kstart + split * chunk;
-    const int we = min(kend, ws + chunk);
+    int ws, we;
+    wave_tiles<T>(kstart, kend, wave, ws, we);
 
     // Fused append: workgroup 0 of every (item, kv head) stores the new rows;
     // no workgroup of this launch reads them from the cache.

@@ -314,13 +314,18 @@ bool use_mfma_decode(int mode, int dtype, int rows_tile_, int head_dim, int64_t 
 }
 
 // Split-K workgroups a decode launch aims at: the context's decode_wgs, else
-// KVRT_TARGET_WGS (512), doubled for int8 layers — their VALU-bound waves
-// (2 groups of 8 keys per pass, 118 VGPRs) need 4 waves per SIMD to hide the
-// dequantise and FMA latencies.
-int target_wgs(const kvrt_config &cfg, int dtype = KVRT_BF16) {
+// KVRT_TARGET_WGS (512), doubled for int8 VALU decodes — their waves (2 groups
+// of 8 keys per pass, 118 VGPRs) need 4 waves per SIMD to hide the dequantise
+// and FMA latencies — and halved, one workgroup per CU, for the bf16 MFMA
+// kernel, whose waves keep whole tiles in flight (64 KB per workgroup at D
+// 128): two per CU read no faster and pay twice the set-up and partials
+// (talker launch, 4 streams x 4160 keys: 16.2 us at 256, 17.1 at 512; 2 x 2112:
+// 9.6 and 9.9; 8 x 4160: 26.7 and 28.0; but the VALU kernel under talker
+// masks, 2 x 1029: 11.4 and 11.1).
+int target_wgs(const kvrt_config &cfg, int dtype = KVRT_BF16, bool mfma = false) {
     static const int v = env_int("KVRT_TARGET_WGS", 512);
     if (cfg.decode_wgs > 0) return cfg.decode_wgs;
-    return dtype == KVRT_INT8 ? 2 * v : v;
+    return mfma ? v / 2 : dtype == KVRT_INT8 ? 2 * v : v;
 }
 // Keys a wave must own at least: one main-loop iteration of the kernel
 // variant (8..32 keys), unless KVRT_MIN_KEYS_PER_WAVE asks for more.
@@ -343,11 +348,13 @@ constexpr int64_t kSplitKeyBucket = KVRT_SPLIT_KEY_BUCKET;
 // Whether a decode merges its workgroup partials in its last workgroup
 // (kvrt_config.decode_merge) instead of a second kernel. AUTO: when the
 // partials of one (item, kv head) total at most KVRT_SINGLE_LAUNCH_BYTES
-// (32 KiB): the merging workgroup reads them all, three dependent memory
+// (12 KiB): the merging workgroup reads them all, three dependent memory
 // round trips after the last partial lands, which costs about what the merge
-// kernel's launch does; beyond that one workgroup's read takes longer.
+// kernel's launch does; beyond that one workgroup's read takes longer. (2 query
+// rows at D 128: 8 KiB 16.2 us in one launch, 17.3 in two; 16 KiB 9.6 and 8.1,
+// 24 KiB 9.7 and 8.2, 32 KiB 10.6 and 8.5.)
 bool single_launch_decode(int mode, bool mfma, int head_dim, int R, int rows, int n_parts) {
-    static const int limit = env_int("KVRT_SINGLE_LAUNCH_BYTES", 32768);
+    static const int limit = env_int("KVRT_SINGLE_LAUNCH_BYTES", 12288);
     if (mode == KVRT_MERGE_SEPARATE || !(mfma || decode_wg_merge(head_dim, R))) return false;
     return mode == KVRT_MERGE_LAST_WG || (int64_t)n_parts * rows * head_dim * 4 <= limit;
 }
@@ -778,7 +785,7 @@ int decode_impl(kvrt_ctx *c, int layer, int n, const int32_t *slots, const kvrt_
     const bool mfma = !talker && use_mfma_decode(c->cfg.decode_kernel, s.dtype, R, D, bucket_keys, s.layout) &&
                       !(pmask && s.layout == KVRT_LAYOUT_PAGED && D >= 512);
     const int mfma_keys = s.dtype == KVRT_INT8 && i8_mfma_dma(D, R) ? kI8MfmaKeys : kMfmaDecodeKeys;
-    const int n_split = choose_splits(target_wgs(c->cfg, mfma ? KVRT_BF16 : s.dtype), n, hkv, max_keys,
+    const int n_split = choose_splits(target_wgs(c->cfg, mfma ? KVRT_BF16 : s.dtype, mfma && s.dtype == KVRT_BF16), n, hkv, max_keys,
                                       mfma ? mfma_keys : keys_per_iteration(D, R, s.dtype, s.layout));
     const int Rw = mfma ? std::max(R, kMfmaDecodeMinRows) : R;  // rows per partial (MFMA tiles are 8 or 16)
     const size_t acc_elems = (size_t)n * hkv * n_split * Rw * D;
@@ -1024,7 +1031,7 @@ int tensor_call_setup(const kvrt_tensor *q, const kvrt_tensor *k, const kvrt_ten
     const int64_t keys = window > 0 ? std::min<int64_t>(lmax, window + qn - 1) : lmax;
     tc.mfma = use_mfma_decode(KVRT_DECODE_AUTO, KVRT_BF16, R, (int)D,
                               (keys + kSplitKeyBucket - 1) / kSplitKeyBucket * kSplitKeyBucket, KVRT_LAYOUT_CONTIG);
-    a.n_split = choose_splits(target, (int)n, (int)hkv, keys,
+    a.n_split = choose_splits(tc.mfma ? target / 2 : target, (int)n, (int)hkv, keys,
                               tc.mfma ? kMfmaDecodeKeys : keys_per_iteration((int)D, R, KVRT_BF16, KVRT_LAYOUT_CONTIG));
     a.n_parts = (tc.mfma || decode_wg_merge((int)D, R)) ? a.n_split / kWaves : a.n_split;
     a.scale_log2 = scale * 1.4426950408889634f;

@@ -131,7 +131,8 @@ typedef struct kvrt_config {
     int32_t pool_seed;    /* PAGED: nonzero = hand out pool pages in an order
                              shuffled with this seed (0 = ascending)          */
     int32_t decode_wgs;   /* split-K decode: target workgroups per launch
-                             (0 = 512, or KVRT_TARGET_WGS). Contexts whose
+                             (0 = 512, or KVRT_TARGET_WGS; int8 twice that,
+                             the bf16 MFMA kernel half). Contexts whose
                              launches run beside another model's on a second
                              stream do better with fewer (e.g. 192)          */
     int32_t decode_kernel; /* KVRT_DECODE_*: which kernel runs bf16 decodes of
@@ -156,7 +157,7 @@ typedef struct kvrt_config {
  * LAST_WG: the last workgroup of each (slot, kv head) to finish merges them
  *   inside the decode launch (one launch per layer); the VALU kernel's
  *   16-row tiles at head_dim 512 (no workgroup partials) always use SEPARATE;
- * AUTO: LAST_WG when a (slot, kv head) has at most 32 KiB of partials (one
+ * AUTO: LAST_WG when a (slot, kv head) has at most 12 KiB of partials (one
  *   workgroup reads them all), SEPARATE otherwise.
  * Every mode gives the same results, bit for bit, when a (slot, kv head) has
  * at most 16 partial workgroups; beyond that the merge order differs. */

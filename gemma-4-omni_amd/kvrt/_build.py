@@ -1,19 +1,22 @@
 """Build libkvrt.so (gfx950) in-tree with hipcc.
 
 The library is compiled from ``csrc/kvrt_kernels.hip`` (kernels),
-``csrc/kvrt_prefill.hip`` (chunked prefill) and ``csrc/kvrt_runtime.hip`` (host
-runtime, C ABI in ``include/kvrt.h``). The
-build also compiles ``csrc/kvrt_coherence_probe.hip`` to assembly (never
-linked) and fails if the coherent-access helpers lower differently from what
+``csrc/kvrt_prefill.hip`` and ``csrc/kvrt_prefill_wide.hip`` (chunked prefill)
+and ``csrc/kvrt_runtime.hip`` (host runtime, C ABI in ``include/kvrt.h``);
+kvrt_pycall.so, the calls that read torch tensors directly, from
+``csrc/kvrt_pycall.cpp`` with the host compiler. The build also compiles
+``csrc/kvrt_coherence_probe.hip`` to assembly (never linked) and fails if the coherent-access helpers lower differently from what
 the single-launch decode merge relies on.
 """
 from __future__ import annotations
 
+import importlib.util
 import json
 import os
 import re
 import shutil
 import subprocess
+import sysconfig
 import tempfile
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
@@ -22,6 +25,7 @@ PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR.parent / "csrc"
 INCLUDE = PKG_DIR.parent.parent / "include"
 LIB_PATH = PKG_DIR / "libkvrt.so"
+CALLS_PATH = PKG_DIR / "kvrt_pycall.so"
 SOURCES = ("kvrt_kernels.hip", "kvrt_prefill.hip", "kvrt_prefill_wide.hip", "kvrt_runtime.hip")
 
 AGPR_SOURCES = ("kvrt_prefill_wide.hip",)
@@ -167,17 +171,33 @@ def check_coherence_lowering() -> None:
                            "decode merge relies on:\n  " + "\n  ".join(errs))
 
 
+def _compile_calls(out: Path) -> None:
+    """kvrt_pycall.so, against the running Python and its torch."""
+    torch = Path(importlib.util.find_spec("torch").submodule_search_locations[0])
+    cxx = os.environ.get("CXX") or shutil.which("g++") or hipcc()
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-unused-function", "-Werror=return-type",
+           f"-I{INCLUDE}", f"-I{sysconfig.get_paths()['include']}", f"-I{torch}/include",
+           f"-I{torch}/include/torch/csrc/api/include", str(CSRC / "kvrt_pycall.cpp"), f"-L{torch}/lib",
+           "-ltorch_python", "-ltorch_cpu", "-lc10", f"-Wl,-rpath,{torch}/lib", "-o", str(out)]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"build of kvrt_pycall.so failed:\n{res.stderr}")
+
+
 def build(verbose: bool = False) -> Path:
     """Compile every HIP source and link libkvrt.so next to this file."""
     with tempfile.TemporaryDirectory(prefix="kvrt_build_") as tmp:
         objs = [Path(tmp) / (Path(s).stem + ".o") for s in SOURCES]
-        with ThreadPoolExecutor(max_workers=len(SOURCES) + 1) as pool:
+        with ThreadPoolExecutor(max_workers=len(SOURCES) + 2) as pool:
             futs = [pool.submit(_compile, CSRC / s, o) for s, o in zip(SOURCES, objs)]
             probe = pool.submit(check_coherence_lowering)
+            tmp_calls = Path(tmp) / CALLS_PATH.name
+            calls = pool.submit(_compile_calls, tmp_calls)
             resources: dict[str, dict[str, str]] = {}
             for f in futs:
                 resources.update(f.result())
             probe.result()
+            calls.result()
         # Every kernel of the hot path must run from registers and LDS: scratch
         # (private segment) use means spilled registers or a by-value kernel
         # argument copied to memory, both of which cost a memory round trip per use.
@@ -191,6 +211,7 @@ def build(verbose: bool = False) -> Path:
         if res.returncode != 0:
             raise RuntimeError(f"link of libkvrt.so failed:\n{res.stderr}")
         shutil.move(str(tmp_lib), str(LIB_PATH))
+        shutil.move(str(tmp_calls), str(CALLS_PATH))
     if verbose:
         print(f"[kvrt] built {LIB_PATH}")
     return LIB_PATH

@@ -6,9 +6,11 @@ PyTorch fallback behind any kvrt entry point.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 from ctypes import POINTER, c_float, c_int32, c_int64, c_uint32, c_uint64, c_void_p
 
-from ._build import LIB_PATH
+from ._build import CALLS_PATH, LIB_PATH
 
 KVRT_ABI_VERSION = 3
 KVRT_MAX_RANK = 4
@@ -213,6 +215,17 @@ def load() -> ctypes.CDLL:
                            "rebuild it")
     _lib = lib
     return lib
+
+
+def load_calls():
+    """Load the native call module; raise if it has not been built."""
+    if not CALLS_PATH.exists():
+        raise RuntimeError(f"{CALLS_PATH.name} not found at {CALLS_PATH}; build it first "
+                           "(python -c 'import __graft_entry__ as g; g.build()')")
+    loader = importlib.machinery.ExtensionFileLoader("kvrt_pycall", str(CALLS_PATH))
+    mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("kvrt_pycall", loader))
+    loader.exec_module(mod)
+    return mod
 
 
 def strerror(code: int) -> str:

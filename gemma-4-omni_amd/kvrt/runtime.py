@@ -96,6 +96,24 @@ def current_stream_handle(device: torch.device) -> int:
 _SLOT_ARRAYS: dict = {}
 
 
+_calls = None
+
+
+def calls():
+    """The native call module (csrc/kvrt_pycall.cpp), loaded once. Its functions
+    return 1, with nothing done, for arguments that need the general path."""
+    global _calls
+    if _calls is None:
+        lib = L.load()
+        mod = L.load_calls()
+        fns = (lib.kvrt_bind_stream, lib.kvrt_append_attend_async, lib.kvrt_attend_decode_async,
+               lib.kvrt_attend_talker_async, lib.kvrt_write_positions_async, lib.kvrt_append_gather_async,
+               lib.kvrt_attend_tensors_async)
+        mod.connect(TalkerMask, *(ctypes.cast(f, ctypes.c_void_p).value for f in fns))
+        _calls = mod
+    return _calls
+
+
 def require_cuda(t: torch.Tensor, name: str) -> None:
     if not t.is_cuda:
         raise ValueError(f"{name} must be a GPU tensor (kvrt has no CPU path)")
@@ -228,6 +246,7 @@ class KVRuntime:
         self.max_q = int(max_q)
         self.block_size = int(block_size)
         self.pool_pages = int(pool_pages)
+        self._call = calls()
         self._ctx = ctypes.c_void_p()
         cfg = L.KvrtConfig()
         cfg.struct_size = ctypes.sizeof(L.KvrtConfig)
@@ -298,6 +317,11 @@ class KVRuntime:
     def _own(self) -> None:
         if threading.get_ident() != self._owner_thread:
             raise RuntimeError("kvrt runtime is confined to the host thread that created it")
+
+    def _bound(self) -> tuple[int, int]:
+        """Context and current stream as the native calls take them (they bind it)."""
+        self._own()
+        return self._ctx.value or 0, current_stream_handle(self.device)
 
     def _bind(self) -> None:
         """Bind the current torch stream (refused while work is in flight on another)."""
@@ -407,6 +431,9 @@ class KVRuntime:
         """
         require_cuda(k, "k")
         require_cuda(v, "v")
+        rc = self._call.write_positions(*self._bound(), layer, slots, positions, k, v)
+        if rc <= 0:
+            return _check(rc, "kvrt_write_positions_async")
         flat = [int(p) for row in positions for p in row]
         if len(flat) != k.shape[0] * k.shape[2]:
             raise ValueError("positions must hold Q entries per slot")
@@ -500,6 +527,11 @@ class KVRuntime:
         spec = self.layers[self._owner(layer)]
         if (q.shape[1] // max(1, spec.kv_heads)) * q.shape[2] > self.DECODE_MAX_ROWS:
             return self.attend_prefill(layer, q, slots, scale, out=out)
+        o = torch.empty_like(q) if out is None else out
+        rc = self._call.attend(*self._bound(), layer, slots, float(scale), q, o)
+        if rc <= 0:
+            _check(rc, "kvrt_attend_decode_async")
+            return o
         q = q.contiguous()
         out = torch.empty_like(q) if out is None else out
         self._bind()
@@ -529,6 +561,11 @@ class KVRuntime:
         """Talker attention of q [n, Hq, Q, D] (Q = 2: prefix then audio query;
         Q = 1: audio query) under one :class:`TalkerMask` per slot."""
         require_cuda(q, "q")
+        o = torch.empty_like(q) if out is None else out
+        rc = self._call.attend_talker(*self._bound(), layer, slots, float(scale), q, o, masks)
+        if rc <= 0:
+            _check(rc, "kvrt_attend_talker_async")
+            return o
         q = q.contiguous()
         out = torch.empty_like(q) if out is None else out
         self._bind()
@@ -548,6 +585,11 @@ class KVRuntime:
                       slots: Sequence[int], scale: float, out: torch.Tensor | None = None) -> torch.Tensor:
         """Fused per-layer decode step: append k, v then attend q."""
         require_cuda(q, "q")
+        o = torch.empty_like(q) if out is None else out
+        rc = self._call.append_attend(*self._bound(), layer, slots, float(scale), q, k, v, o)
+        if rc <= 0:
+            _check(rc, "kvrt_append_attend_async")
+            return o
         q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
         out = torch.empty_like(q) if out is None else out
         self._bind()
@@ -621,6 +663,11 @@ class KVRuntime:
         mask = out[2] if len(out) > 2 else None
         if mask is not None:
             require_cuda(mask, "out mask")
+        if start_pos is None:
+            rc = self._call.append_gather(*self._bound(), layer, slots, k, v, out_k, out_v, mask)
+            if rc <= 0:
+                _check(rc, "kvrt_append_gather_async")
+                return out_k, out_v, mask
         self._bind()
         arr, n = self._slots(slots)
         sp = None if start_pos is None else (ctypes.c_int32 * n)(*[int(x) for x in start_pos])
@@ -776,6 +823,12 @@ def attend_tensors(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, lengths: t
     lib = L.load()
     for t, name in ((q, "q"), (k, "k"), (v, "v"), (lengths, "lengths")):
         require_cuda(t, name)
+    if prefix_attention is None:
+        o = torch.empty_like(q) if out is None else out
+        rc = calls().attend_tensors(current_stream_handle(q.device), float(scale), int(window), q, k, v, lengths, o)
+        if rc <= 0:
+            _check(rc, "kvrt_attend_tensors_async")
+            return o
     q = q.contiguous()
     lengths = lengths.to(torch.int32).contiguous()
     out = torch.empty_like(q) if out is None else out

@@ -279,13 +279,20 @@ constexpr int kMaxWgPerHead = 64;
 // head_dim 512, 8 rows at head_dim <= 256 over at least kMfmaDecodeMinKeys8
 // visible keys, and 1-4 rows over as many keys where the tiles stream through
 // the LDS DMA ring (mfma_decode_dma) — the shapes where the VALU kernel's
-// dot products and P.V products make it compute-bound. Short 8-row decodes (a
-// 512-key sliding window) stay on the VALU kernel: latency-bound either way,
-// and lighter on a concurrent stream. `keys` is the launch's key count
-// rounded up to the split bucket, so the choice, like the split count, stays
-// fixed within a bucket.
+// dot products and P.V products make it compute-bound. Shorter ones are a
+// chain of latencies: a wave's 8 rows cost the VALU kernel ~2 us of dot
+// products and reductions between its load and its partial, and four times
+// the partials (4 keys per wave, not 16) to merge. A single stream's, whose
+// step waits for every one of them, run on the MFMA kernel too (8 rows, D 256
+// x 512 ring keys: 9.3 -> 7.5 us with the merge; D 128 x 130 9.5 -> 6.5; 4
+// rows, D 128 x 513 7.6 -> 6.5; but 4 rows at D 256 x 33 7.3 and 7.4, 2 rows
+// at D 64 x 1100 5.9 and 6.2). Short batches stay on the VALU kernel, which
+// kvrt_counters.mfma_decodes reports of them: 10.3 against 8.0 us with 4
+// streams of that ring, and 0.7 % of a two-model step. `keys` is the launch's
+// key count rounded up to the split bucket, so the choice, like the split
+// count, stays fixed within a bucket.
 constexpr int64_t kMfmaDecodeMinKeys8 = 2048;
-bool use_mfma_decode(int mode, int dtype, int rows_tile_, int head_dim, int64_t keys, int layout) {
+bool use_mfma_decode(int mode, int dtype, int rows_tile_, int head_dim, int64_t keys, int layout, int n_items) {
     if (mode == KVRT_DECODE_VALU) return false;
     // int8 (PAGED): AUTO keeps the VALU kernel. A forced MFMA decode runs
     // the int8 ring kernel at head_dim 64 / 128 (i8_mfma_dma), the register-
@@ -307,10 +314,11 @@ bool use_mfma_decode(int mode, int dtype, int rows_tile_, int head_dim, int64_t 
         static const char *env = std::getenv("KVRT_MFMA_SMALL_ROWS");
         static const bool small = !env || std::atoi(env) != 0;
         static const int64_t min_keys_small = env_int("KVRT_MFMA_SMALL_MIN_KEYS", (int)kMfmaDecodeMinKeys8);
-        return mode == KVRT_DECODE_MFMA ||
+        return mode == KVRT_DECODE_MFMA || (small && n_items == 1 && rows_tile_ == 4 && head_dim <= 128) ||
                (small && mfma_decode_dma(head_dim, rows_tile_, dtype, layout) && keys >= min_keys_small);
     }
-    return mode == KVRT_DECODE_MFMA || rows_tile_ >= 16 || head_dim >= 512 || keys >= kMfmaDecodeMinKeys8;
+    return mode == KVRT_DECODE_MFMA || rows_tile_ >= 16 || head_dim >= 512 || n_items == 1 ||
+           keys >= kMfmaDecodeMinKeys8;
 }
 
 // Split-K workgroups a decode launch aims at: the context's decode_wgs, else
@@ -782,7 +790,7 @@ int decode_impl(kvrt_ctx *c, int layer, int n, const int32_t *slots, const kvrt_
     const int64_t bucket_keys = (max_keys + kSplitKeyBucket - 1) / kSplitKeyBucket * kSplitKeyBucket;
     const PrefixMask *pmask = talker ? nullptr : launch_masks(c, n, slots);
     // the MFMA kernel's PAGED D 512 variant has no registers for a mask
-    const bool mfma = !talker && use_mfma_decode(c->cfg.decode_kernel, s.dtype, R, D, bucket_keys, s.layout) &&
+    const bool mfma = !talker && use_mfma_decode(c->cfg.decode_kernel, s.dtype, R, D, bucket_keys, s.layout, n) &&
                       !(pmask && s.layout == KVRT_LAYOUT_PAGED && D >= 512);
     const int mfma_keys = s.dtype == KVRT_INT8 && i8_mfma_dma(D, R) ? kI8MfmaKeys : kMfmaDecodeKeys;
     const int n_split = choose_splits(target_wgs(c->cfg, mfma ? KVRT_BF16 : s.dtype, mfma && s.dtype == KVRT_BF16), n, hkv, max_keys,
@@ -1030,7 +1038,7 @@ int tensor_call_setup(const kvrt_tensor *q, const kvrt_tensor *k, const kvrt_ten
     const int R = rows_tile(rows);
     const int64_t keys = window > 0 ? std::min<int64_t>(lmax, window + qn - 1) : lmax;
     tc.mfma = use_mfma_decode(KVRT_DECODE_AUTO, KVRT_BF16, R, (int)D,
-                              (keys + kSplitKeyBucket - 1) / kSplitKeyBucket * kSplitKeyBucket, KVRT_LAYOUT_CONTIG);
+                              (keys + kSplitKeyBucket - 1) / kSplitKeyBucket * kSplitKeyBucket, KVRT_LAYOUT_CONTIG, (int)n);
     a.n_split = choose_splits(tc.mfma ? target / 2 : target, (int)n, (int)hkv, keys,
                               tc.mfma ? kMfmaDecodeKeys : keys_per_iteration((int)D, R, KVRT_BF16, KVRT_LAYOUT_CONTIG));
     a.n_parts = (tc.mfma || decode_wg_merge((int)D, R)) ? a.n_split / kWaves : a.n_split;

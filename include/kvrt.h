@@ -142,8 +142,9 @@ typedef struct kvrt_config {
 } kvrt_config;
 
 /* kvrt_config.decode_kernel. AUTO: MFMA for bf16 decodes of 16 rows per kv
- * head, and of 8 rows at head_dim 512 or over >= 2048 visible keys; the VALU
- * kernel otherwise (int8 included). VALU / MFMA force one kernel for every
+ * head, of 8 rows at head_dim 512 or over >= 2048 visible keys, and a single
+ * slot's of 8 rows (4 to head_dim 128) over any keys; the VALU kernel
+ * otherwise (int8 included). VALU / MFMA force one kernel for every
  * eligible decode (MFMA: bf16 with 8 or 16 rows per kv head, or int8 PAGED
  * with up to 8; not the talker masks; other decodes always run on the VALU
  * kernel). */

@@ -51,3 +51,29 @@ def test_tiles_left_over(layout, d, hq, qn, wgs):
             np.testing.assert_allclose(_np(out[0]), ref, rtol=2.0 ** -8, atol=ATOL, err_msg=f"{n} keys")
         assert rt.health() == 0
         assert rt.counters()["mfma_decodes"] == 3
+
+
+@pytest.mark.parametrize("d,hq,qn,streams,mfma", [(256, 8, 1, 1, True), (256, 5, 1, 1, True), (64, 4, 2, 1, True),
+                                                  (128, 4, 1, 1, True), (128, 3, 1, 1, True), (256, 4, 1, 1, False),
+                                                  (128, 2, 1, 1, False), (256, 8, 1, 2, False)])
+@pytest.mark.parametrize("keys", [1, 33, 513])
+def test_short_decodes_by_stream_count(d, hq, qn, streams, mfma, keys):
+    """Under 2048 keys a single stream's 8 rows, and 4 rows to head_dim 128, run
+    on MFMA tiles; fewer rows and batches do not."""
+    from kvrt import KVRuntime, LayerSpec
+
+    gen = torch.Generator().manual_seed(d + hq + keys)
+    bf = lambda shape: torch.randn(shape, generator=gen).to(torch.bfloat16)
+    rt = KVRuntime([LayerSpec(kv_heads=1, head_dim=d)], streams, keys + 4, max_q=qn, device="cuda")
+    orc = O.OracleCache([O.OracleLayer(1, d, 0)], streams)
+    for s in range(streams):
+        k, v = bf((1, 1, keys, d)), bf((1, 1, keys, d))
+        rt.import_(s, 0, k.cuda(), v.cuda())
+        orc.append(s, 0, _np(k[0]), _np(v[0]))
+    q, k, v = bf((streams, hq, qn, d)), bf((streams, 1, qn, d)), bf((streams, 1, qn, d))
+    out = rt.append_attend(0, q.cuda(), k.cuda(), v.cuda(), list(range(streams)), 0.25 / math.sqrt(d))
+    for s in range(streams):
+        orc.append(s, 0, _np(k[s]), _np(v[s]))
+        np.testing.assert_allclose(_np(out[s]), orc.attend(s, 0, _np(q[s]), 0.25 / math.sqrt(d)), rtol=2.0 ** -8,
+                                   atol=ATOL)
+    assert rt.counters()["mfma_decodes"] == int(mfma) and rt.health() == 0

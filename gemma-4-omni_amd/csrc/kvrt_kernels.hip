@@ -2177,7 +2177,8 @@ __global__ __launch_bounds__(512) void prefix_pack_kernel(PrefixPackArgs a) {
 // 16-B units per thread of head y of layer e's K (j = 0) or V rows. One pass
 // over the slot instead of a fill and a copy per layer and tensor, HBM-bound:
 // 28 layers of 8 heads x 1024 rows x 128, 700 of them imported, took 57 fills
-// (2.2 us each) and 28 copies (4.3 us), now one launch of 46 us (198 MB).
+// (2.2 us each) and 28 copies (4.3 us): 300 us a session, 50 us in this launch
+// (198 MB).
 constexpr int kOpenUnits = 4;
 __global__ __launch_bounds__(256) void open_slot_kernel(OpenArgs a) {
     const OpenLayer &L = a.l[blockIdx.z >> 1];

@@ -207,17 +207,11 @@ __global__ __launch_bounds__(64 * RW * KS) void prefill_kernel(PrefillArgs a) {
     const int pq = base_pos + qr;
     // the workgroup's keys: from its first query's window to its last query;
     // with a key split, range ks of them in whole blocks
-    int kend = base_pos + ql + 1;
-    int kstart = a.window > 0 ? max(0, base_pos + qf - a.window + 1) : 0;
+    const KeyRange range = prefill_range(base_pos, qf, ql, a.window, nks, ks, kPfKeys);
+    const int kstart = range.kstart, kend = range.kend;
     const int wkend = base_pos + wql + 1;  // the same for this wave's rows
     const int wkstart = a.window > 0 ? max(0, base_pos + wqf - a.window + 1) : 0;
-    if (nks > 1) {
-        const int span = (kend - kstart + nks - 1) / nks;
-        const int len = (span + kPfKeys - 1) / kPfKeys * kPfKeys;
-        const int k0 = kstart + ks * len;
-        kend = min(kend, k0 + len);
-        kstart = min(k0, kend);
-    }
+    const int ngroups = (kend - kstart + kPfKeys * KS - 1) / (kPfKeys * KS);  // <= 0: no keys, nothing is fetched
     // keys this lane's row sees: [klo, khi] (none if the lane has no row)
     const int khi = qvalid ? min(kend - 1, pq) : -1;
     const int klo = a.window > 0 ? pq - a.window + 1 : 0;
@@ -259,7 +253,8 @@ __global__ __launch_bounds__(64 * RW * KS) void prefill_kernel(PrefillArgs a) {
         return load_page_window(a.kv, slot, min(t, kend - 1) >> a.kv.block_shift, lane);
     };
     int pages = 0;  // of the block at kt
-    if constexpr (LAYOUT == KVRT_LAYOUT_PAGED) pages = load_pages(kt);
+    if constexpr (LAYOUT == KVRT_LAYOUT_PAGED)
+        if (ngroups > 0) pages = load_pages(kt);  // kend > kstart >= 0
     auto next_fetch = [&]() __attribute__((always_inline)) {
         const int t0 = min(kt, kend - 1);
         Fetch f;
@@ -299,7 +294,6 @@ __global__ __launch_bounds__(64 * RW * KS) void prefill_kernel(PrefillArgs a) {
         }
     };
 
-    const int ngroups = (kend - kstart + kPfKeys * KS - 1) / (kPfKeys * KS);
     Fetch kf{}, vf{};
     if (ngroups > 0) {  // the first K blocks
         kf = next_fetch();

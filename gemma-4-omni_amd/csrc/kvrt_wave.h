@@ -6,6 +6,7 @@
 
 #include "kvrt_device.h"
 #include "kvrt_internal.h"
+#include "kvrt_range.h"
 
 namespace kvrt {
 
@@ -99,10 +100,10 @@ __device__ __forceinline__ int umod_uniform(int x, int d) {
 }
 
 // A wave's window of page-table entries: lane i holds the entry of logical
-// page win0 + i of the slot (-1 past the table).
+// page win0 + i of the slot (-1 outside the table).
 __device__ __forceinline__ int load_page_window(const KVView &v, int slot, int win0, int lane) {
     const int lp = win0 + lane;
-    return lp < v.pt_stride ? v.page_table[(int64_t)slot * v.pt_stride + lp] : -1;
+    return page_in_table(lp, v.pt_stride) ? v.page_table[(int64_t)slot * v.pt_stride + lp] : -1;
 }
 // Element offset of row pos of a head on a page; -1 if the page is unmapped
 // or out of the pool.

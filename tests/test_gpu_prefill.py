@@ -262,3 +262,40 @@ def test_prefill_at_the_benchmark_shapes_on_sampled_rows(name, n, hq, hkv, d, qn
         ref = O.attend(to_np(q[s])[:, rows], ks[s], vs[s], np.array([L - qn + i for i in rows]), scale, window)
         worst = max(worst, float(np.abs(to_np(out[s])[:, rows] - ref).max()))
     assert worst <= ATOL, worst
+
+
+@pytest.mark.parametrize("hq,hkv,d,window,layout,prefix", [
+    (8, 2, 64, 0, "paged", 1500), (16, 8, 128, 0, "paged", 60), (8, 1, 512, 0, "paged", 700), (8, 1, 256, 90, "paged", 200),
+    (16, 8, 128, 0, "contig", 900), (8, 1, 256, 512, "ring", 300)])
+def test_captured_prefill_replayed_below_its_query_count(hq, hkv, d, window, layout, prefix):
+    """A captured chunk replayed after a rollback to fewer rows than queries:
+    query i sits at position length - Q + i, and those before position 0 see no
+    keys (zeros), whatever the other slots hold. The page arithmetic itself is
+    tests/test_prefill_range.py's."""
+    qn, left = 70, (7, 33)
+    rt, orc, q = _setup(hq, hkv, d, window, layout, [prefix, prefix], qn, seed=d + hq)
+    scale = 1.0 / math.sqrt(d)
+    q, out = q.cuda(), torch.empty(q.shape, dtype=torch.bfloat16, device="cuda")
+    rt.attend_prefill(0, q, [0, 1], scale, out=out)
+    rt.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        rt.attend_prefill(0, q, [0, 1], scale, out=out)
+    rt.sync_lengths()
+    if layout == "ring":  # the rows of [0, left) are no longer stored: only an empty slot can be rolled back to
+        left = (0, 0)
+    for s, n in enumerate(left):
+        rt.truncate(s, n)
+        orc.truncate(s, 0, n)
+    rt.synchronize()
+    for _ in range(3):
+        out.fill_(7.0)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        for s, n in enumerate(left):
+            assert not out[s, :, :qn - n].any()
+            if n:
+                ref = orc.attend(s, 0, to_np(q[s])[:, qn - n:], scale)
+                assert float(np.abs(to_np(out[s])[:, qn - n:] - ref).max()) <= ATOL
+    assert rt.health() == 0

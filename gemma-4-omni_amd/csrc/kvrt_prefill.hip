@@ -52,7 +52,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a, int D
             O.w = fmaf(v[u].w, w, O.w);
         }
     }
-    const bool any = L > 0.f;
+    const bool any = !(L == 0.f);  // no key: 0; a NaN sum stays NaN, as without a split
     const uint2 packed = make_uint2(pack_bf16x2(any ? O.x / L : 0.f, any ? O.y / L : 0.f),
                                     pack_bf16x2(any ? O.z / L : 0.f, any ? O.w / L : 0.f));
     *reinterpret_cast<uint2 *>(a.out + row * D + d) = packed;

@@ -299,3 +299,24 @@ def test_captured_prefill_replayed_below_its_query_count(hq, hkv, d, window, lay
                 ref = orc.attend(s, 0, to_np(q[s])[:, qn - n:], scale)
                 assert float(np.abs(to_np(out[s])[:, qn - n:] - ref).max()) <= ATOL
     assert rt.health() == 0
+
+
+@pytest.mark.parametrize("d,hq,hkv,prefix,qn,window,split", [
+    (512, 8, 1, 236, 64, 0, True), (512, 8, 1, 20, 64, 0, False), (256, 8, 1, 1500, 30, 0, True),
+    (256, 8, 1, 100, 200, 512, False), (128, 16, 8, 2000, 20, 0, True), (128, 16, 8, 100, 60, 0, False)])
+@pytest.mark.parametrize("where", ["k", "q"])
+def test_nan_stays_nan_with_and_without_a_key_split(d, hq, hkv, prefix, qn, window, split, where):
+    """A NaN in a key that every query sees makes their rows NaN, one in a query
+    its own row, whichever launch shape the chunk takes."""
+    rt, _, q = _setup(hq, hkv, d, window, "contig", [prefix], qn, seed=3)
+    want = torch.zeros((1, hq, qn, d), dtype=torch.bool)
+    if where == "k":
+        rt.storage(0)[0][0, 0, prefix - 5, 3] = float("nan")  # kv head 0, seen by all queries
+        want[:, :hq // hkv] = True
+    else:
+        q[0, 1, qn // 2, 7] = float("nan")
+        want[0, 1, qn // 2] = True
+    launches = rt.counters()["launches"]
+    out = rt.attend_prefill(0, q.cuda(), [0], 1.0 / math.sqrt(d))
+    assert rt.counters()["launches"] == launches + (2 if split else 1)
+    assert torch.equal(out.isnan().cpu(), want)

@@ -300,6 +300,7 @@ struct PrefillArgs {
     int32_t window;
     int32_t row_waves;      // 32-row blocks (q heads x queries) per workgroup
     int32_t key_parts;      // waves per row block, splitting the keys
+    int32_t short_heads;    // > 0: kvrt_prefill_short.hip, that many q heads x row_waves 16-query blocks per workgroup
     int32_t n_ksplit;       // key ranges per row block; > 1: partials to part_o / part_ml
     float *part_o;          // [n, Hq, Q, n_ksplit, D] unnormalised outputs
     float2 *part_ml;        // [n, Hq, Q, n_ksplit] (running max in log2 units, sum)
@@ -396,6 +397,7 @@ hipError_t launch_decode_talker(const TalkerArgs &a, int head_dim, int rows_per_
 // Chunked-prefill attention on MFMA (bf16 CONTIG / RING / PAGED layers).
 hipError_t launch_prefill(const PrefillArgs &a, int head_dim, hipStream_t s);
 hipError_t launch_prefill_wide(const PrefillArgs &a, int head_dim, hipStream_t s);  // head_dim 256, 512
+hipError_t launch_prefill_short(const PrefillArgs &a, int head_dim, hipStream_t s);  // head_dim 128, few keys
 constexpr int kPfKeys = 32;  // keys per staged block of the prefill kernel
 hipError_t launch_set_lens(const SetLenArgs &a, hipStream_t s);
 hipError_t launch_set_pages(int32_t *pt, int n, const int32_t *idx, const int32_t *val,

@@ -294,11 +294,25 @@ __global__ __launch_bounds__(64 * RW * KS) void prefill_kernel(PrefillArgs a) {
         }
     };
 
+    // At head_dim 256 the first V blocks are fetched with the first K blocks, a
+    // round trip earlier than beside the first K Q^T (Q 9 over 9 6.9 -> 6.6 us).
+    // At 512 that would hold the first scores up by 32 KiB more, and below, where
+    // several workgroups share a CU, it is no faster.
+    constexpr bool V_FIRST = D == 256;
     Fetch kf{}, vf{};
-    if (ngroups > 0) {  // the first K blocks
+    // Parts with a block in the range; the others fetch nothing ahead of the
+    // loop and add nothing at its end.
+    const int nparts = KS == 1 ? 1 : max(1, min(KS, (kend - kstart + kPfKeys - 1) / kPfKeys));
+    if (ngroups > 0) {  // the first K and V blocks
         kf = next_fetch();
+        vf = kf;
+        if (part < nparts) {
 #pragma unroll
-        for (int i = 0; i < IPW; ++i) fetch(std::false_type{}, kf, 0, i);
+            for (int i = 0; i < IPW; ++i) fetch(std::false_type{}, kf, 0, i);
+            if constexpr (V_FIRST)
+#pragma unroll
+                for (int i = 0; i < IPW; ++i) fetch(std::true_type{}, vf, 0, i);
+        }
     }
 
     // A negative scale is moved into q's sign bits (exact, below), so that the
@@ -343,11 +357,12 @@ __global__ __launch_bounds__(64 * RW * KS) void prefill_kernel(PrefillArgs a) {
     f32x16_t s;         // scores of the block after it
     int cur = 0;  // the iteration
     // The iteration's DMAs (the K blocks of group it + 2, then the V blocks of
-    // it + 1), spread over SPAN steps: the first half of all steps, at head_dim
-    // 512 of the P V ones, whose MFMAs leave the most issue slots free. They are issued past the last
-    // group too (clamped to its last key): a branch around each costs more
-    // than the DMAs it would save.
-    constexpr int DMA0 = D == 512 ? NK : 0, SPAN = D == 512 ? NP / 2 : (NK + NP) / 2;
+    // it + 1), spread over SPAN steps: those of K Q^T, at head_dim 512 the first
+    // half of the P V ones, whose MFMAs leave the most issue slots free. Past
+    // the last group they read its last key (a branch around each costs more
+    // than the DMAs it would save); up to head_dim 256 the last iteration, which
+    // has no K Q^T, issues none, and the kernel's end waits for none.
+    constexpr int DMA0 = D == 512 ? NK : 0, SPAN = D == 512 ? NP / 2 : NK;
     auto dma_at = [&](auto c_c) __attribute__((always_inline)) {
         constexpr int c = decltype(c_c)::value - DMA0;
         if constexpr (c >= 0 && c < SPAN)
@@ -499,13 +514,15 @@ __global__ __launch_bounds__(64 * RW * KS) void prefill_kernel(PrefillArgs a) {
             x = make_uint4(x.x ^ flip, x.y ^ flip, x.z ^ flip, x.w ^ flip);
             asm volatile("" : "+v"(x.x), "+v"(x.y), "+v"(x.z), "+v"(x.w));
         }
-        // the first V blocks and the second K blocks, in flight beside the first K Q^T
-        vf = kf;
-        kf = next_fetch();
+        // the second K blocks, in flight beside the first K Q^T
+        if constexpr (!V_FIRST)
 #pragma unroll
-        for (int i = 0; i < IPW; ++i) fetch(std::true_type{}, vf, 0, i);
+            for (int i = 0; i < IPW; ++i) fetch(std::true_type{}, vf, 0, i);
+        if (ngroups > 1) {
+            kf = next_fetch();
 #pragma unroll
-        for (int i = 0; i < IPW; ++i) fetch(std::false_type{}, kf, 1, i);
+            for (int i = 0; i < IPW; ++i) fetch(std::false_type{}, kf, 1, i);
+        }
         __syncthreads();
         if (jlo == 0 && jhi > 0) {
             score_steps(part, 0, std::true_type{});
@@ -528,7 +545,7 @@ __global__ __launch_bounds__(64 * RW * KS) void prefill_kernel(PrefillArgs a) {
                 score_steps(kblk, vblk, std::false_type{});
                 mask(key0(it + 1));
             } else {
-                StaticFor<0, NK>::run(dma_at);
+                if (it + 1 < ngroups) StaticFor<0, NK>::run(dma_at);
 #pragma unroll
                 for (int u = 0; u < PV; ++u) vx[u] = vop(vblk, u % NB, u / NB);
             }
@@ -635,11 +652,12 @@ __global__ __launch_bounds__(64 * RW * KS) void prefill_kernel(PrefillArgs a) {
 #pragma unroll
         for (int b0 = 0; b0 < NB; b0 += BS) {
             if (b0 > 0) __syncthreads();
+            if (part < nparts)
 #pragma unroll
-            for (int b = 0; b < BS; ++b)
+                for (int b = 0; b < BS; ++b)
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    mine[(b * 4 + i) * 64] = make_float4(o[b0 + b][4 * i] * w, o[b0 + b][4 * i + 1] * w,
+                    for (int i = 0; i < 4; ++i)
+                        mine[(b * 4 + i) * 64] = make_float4(o[b0 + b][4 * i] * w, o[b0 + b][4 * i + 1] * w,
                                                          o[b0 + b][4 * i + 2] * w, o[b0 + b][4 * i + 3] * w);
             __syncthreads();
             if (wlive) {
@@ -649,12 +667,14 @@ __global__ __launch_bounds__(64 * RW * KS) void prefill_kernel(PrefillArgs a) {
 #pragma unroll
                     for (int e = 0; e < 2; ++e) x[e] = xo(rw)[(b * 4 + i + e) * 64];
 #pragma unroll
-                    for (int p = 1; p < KS; ++p)
+                    for (int p = 1; p < KS; ++p) {
+                        if (p >= nparts) break;
 #pragma unroll
                         for (int e = 0; e < 2; ++e) {
                             const float4 y = xo(p * RW + rw)[(b * 4 + i + e) * 64];
                             x[e] = make_float4(x[e].x + y.x, x[e].y + y.y, x[e].z + y.z, x[e].w + y.w);
                         }
+                    }
                     if (nks == 1) {
                         store_bf16(b0 + b, i, x[0], x[1]);
                     } else if (evalid) {
@@ -668,25 +688,22 @@ __global__ __launch_bounds__(64 * RW * KS) void prefill_kernel(PrefillArgs a) {
     }
 }
 
-template <int D, int RW, int KS, int NS>
-static hipError_t launch_prefill_shape(const PrefillArgs &a, hipStream_t s) {
+template <int D, int RW, int KS, int NS, int LAYOUT>
+static hipError_t launch_prefill_layout(const PrefillArgs &a, hipStream_t s) {
     const int64_t rows = (int64_t)a.group * a.qn;
     const dim3 grid(a.n_ksplit * a.kv.kv_heads, a.n_items, (unsigned)((rows + 32 * RW - 1) / (32 * RW)));
-    const dim3 block(64 * RW * KS);
-    switch (a.kv.layout) {
-        case KVRT_LAYOUT_CONTIG:
-            hipLaunchKernelGGL((prefill_kernel<D, KVRT_LAYOUT_CONTIG, RW, KS, NS>), grid, block, 0, s, a);
-            break;
-        case KVRT_LAYOUT_RING:
-            hipLaunchKernelGGL((prefill_kernel<D, KVRT_LAYOUT_RING, RW, KS, NS>), grid, block, 0, s, a);
-            break;
-        case KVRT_LAYOUT_PAGED:
-            hipLaunchKernelGGL((prefill_kernel<D, KVRT_LAYOUT_PAGED, RW, KS, NS>), grid, block, 0, s, a);
-            break;
-        default:
-            return hipErrorInvalidValue;
-    }
+    hipLaunchKernelGGL((prefill_kernel<D, LAYOUT, RW, KS, NS>), grid, dim3(64 * RW * KS), 0, s, a);
     return hipGetLastError();
+}
+
+template <int D, int RW, int KS, int NS>
+static hipError_t launch_prefill_shape(const PrefillArgs &a, hipStream_t s) {
+    switch (a.kv.layout) {
+        case KVRT_LAYOUT_CONTIG: return launch_prefill_layout<D, RW, KS, NS, KVRT_LAYOUT_CONTIG>(a, s);
+        case KVRT_LAYOUT_RING: return launch_prefill_layout<D, RW, KS, NS, KVRT_LAYOUT_RING>(a, s);
+        case KVRT_LAYOUT_PAGED: return launch_prefill_layout<D, RW, KS, NS, KVRT_LAYOUT_PAGED>(a, s);
+        default: return hipErrorInvalidValue;
+    }
 }
 
 }  // namespace kvrt

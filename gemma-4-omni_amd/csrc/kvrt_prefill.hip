@@ -74,6 +74,7 @@ hipError_t launch_prefill(const PrefillArgs &a, int head_dim, hipStream_t s) {
     if (a.group <= 0 || a.qn <= 0 || a.n_items <= 0) return hipErrorInvalidValue;
     if (a.n_ksplit < 1 || (a.n_ksplit > 1 && (!a.part_o || !a.part_ml))) return hipErrorInvalidValue;
     if (a.kv.layout == KVRT_LAYOUT_RING && a.kv.rows < kPfKeys) return hipErrorInvalidValue;
+    if (a.short_heads > 0) return launch_prefill_short(a, head_dim, s);
     const int rw = a.row_waves, ks = a.key_parts;
     hipError_t e = hipErrorInvalidValue;
     const auto shapes = [&](auto d_c) {
@@ -81,7 +82,10 @@ hipError_t launch_prefill(const PrefillArgs &a, int head_dim, hipStream_t s) {
         if (rw == 4 && ks == 1) return launch_prefill_shape<D, 4, 1, 2>(a, s);
         if (rw == 2 && ks == 2) return launch_prefill_shape<D, 2, 2, 2>(a, s);
         if (rw == 2 && ks == 4) return launch_prefill_shape<D, 2, 4, 2>(a, s);
-        if (rw == 1 && ks == 4) return launch_prefill_shape<D, 1, 4, 2>(a, s);
+        if (rw == 1 && ks == 4 && a.kv.layout == KVRT_LAYOUT_CONTIG)
+            return launch_prefill_layout<D, 1, 4, 2, KVRT_LAYOUT_CONTIG>(a, s);
+        if (rw == 1 && ks == 4 && a.kv.layout == KVRT_LAYOUT_RING)
+            return launch_prefill_layout<D, 1, 4, 2, KVRT_LAYOUT_RING>(a, s);
         return hipErrorInvalidValue;
     };
     if (head_dim == 64) {

@@ -2134,18 +2134,64 @@ int kvrt_attend_prefill_async(kvrt_ctx *c, int32_t layer, int32_t n, const int32
         // so are they where two parts would not have a block each
         if (block_keys > 64 && wgs(2) <= (s.window > 0 ? 384 : 512)) rw = 2, parts = 2;
         min_keys = 80, split_keys = 400;
-    } else if (D <= 128) {
-        // four parts while one round of workgroups takes the grid (Hq 16, one
-        // stream x Q 512: 10.0 us, two parts 12.2; x Q 800 over 2000: 35.1, 40.8),
-        // two up to two rounds of four row blocks (4 x Q 512: 15.4 us, four
-        // parts 20.4), none beyond (4 x Q 1400: 98.7 us, two parts 102.6). A
-        // PAGED row's address costs a lane more than its DMA: two row blocks
-        // share the fetching, and a split pays with half the keys.
-        if (wgs(1) <= 256 && s.layout != KVRT_LAYOUT_PAGED) rw = 1, parts = 4;
-        else if (wgs(2) < 256) rw = 2, parts = 4;
+    } else if (D <= 128 && s.layout == KVRT_LAYOUT_PAGED) {
+        // A row's address costs a lane more than its DMA: two row blocks share
+        // the fetching, and a split pays with half the keys. Few keys take no
+        // more parts than they have blocks (Hq 16 x Q 12 over 12: 4.6 us, two
+        // parts 5.5, four 5.7; Q 40 over 60: 6.4, four parts 7.2; over 220:
+        // 11.1, two parts 11.2).
+        if (block_keys <= 32) rw = 4, parts = 1;
+        else if (wgs(2) < 256) rw = 2, parts = block_keys <= 160 ? 2 : 4;
         else if (wgs(4) < 512) rw = 2, parts = 2;
-        min_keys = s.layout == KVRT_LAYOUT_PAGED ? 180 : 360;
-        split_keys = s.layout == KVRT_LAYOUT_PAGED ? 250 : 500;
+        min_keys = 180, split_keys = 250;
+    } else if (D <= 128) {
+        // Few keys: 16-query tiles (kvrt_prefill_short.hip), whose chain per
+        // tile is half as long. 16-query tiles against the shape chosen below,
+        // us (graph replays, warm rows):
+        // up to one round of row blocks, D 128: Q 64 over 64 4.2 and 5.3, over
+        // 164 5.8 and 6.9; Q 40 over 300 7.4 and 7.7, over 400 9.3 and 8.3
+        // (more than one 16-query workgroup per CU: 8 heads of their own, 2 x
+        // Q 300 over 300, 8.1 and 7.8).
+        // Three or four heads of a group fill a workgroup's eight waves and the
+        // line lies lower: 3 heads x Q 40 over 150 6.6 and 7.1, over 200 7.4
+        // and 7.0; 4 heads over 40 4.9 and 5.2, over 100 5.9 and 5.7.
+        // D 64: Q 40 over 150 4.4 and 5.3, over 220 5.0 and 5.2.
+        // In a second round (4 x Q 200): over 300 8.7 and 9.5, over 550 11.9 and
+        // 12.5; D 64 over 400 7.3 and 8.1.
+        // Beyond, while the 16-query grid is at most four workgroups per CU: 16
+        // x Q 100 over 160 10.7 and 10.9, over 320 14.5 and 14.1; past that (32
+        // x Q 100 over 100) 15.0 and 11.1.
+        int heads = 1;  // q heads of a workgroup
+        for (int h = 2; h <= std::min(group, 4); ++h)
+            if (group % h == 0) heads = h;
+        const int64_t blocks = wgs(1), wgs16 = (qn + 15) / 16 * hkv * (group / heads) * n;
+        int short_keys = 0;
+        if (D == 128 && blocks <= 256) short_keys = heads == 3 ? 160 : heads > 3 ? 64 : wgs16 <= 256 ? 320 : 208;
+        else if (D == 128 && blocks <= 512) short_keys = heads <= 2 ? 576 : 320;
+        else if (D == 128) short_keys = wgs16 <= 1024 ? 224 : 0;
+        else if (blocks <= 256) short_keys = heads <= 3 ? 160 : 64;
+        else if (blocks <= 512 && heads <= 2) short_keys = 416;
+        if (block_keys <= short_keys && ksplit_env < 2) {
+            a.short_heads = heads;
+            // two query blocks on the same tiles from two workgroups per CU on
+            const bool pair = wgs16 >= 512;
+            rw = pair ? 2 : 1;
+            parts = pair && heads > 2 ? 1 : 2;
+        } else if (blocks <= (D == 64 ? 512 : 256)) {
+            // four parts while one round of workgroups (at D 64 two per CU)
+            // takes the grid (Hq 16, one stream x Q 512: 8.8 us, two parts
+            // 10.9; D 64 x Q 450, 2 streams, 7.6 and 8.6)
+            rw = 1, parts = 4;
+        } else if (D == 128 && wgs(2) < 256) {
+            // (3 streams x Q 274 over 947: 16.9 us, two parts 17.4)
+            rw = 2, parts = 4;
+        } else if (wgs(4) < 512) {
+            // two parts up to two rounds of four row blocks (4 x Q 512: 15.4
+            // us, four parts 20.4), none beyond (4 x Q 1400: 98.7 us, two
+            // parts 102.6)
+            rw = 2, parts = 2;
+        }
+        min_keys = 160, split_keys = 500;
     }
     a.row_waves = rw;
     a.key_parts = parts;
@@ -2156,7 +2202,7 @@ int kvrt_attend_prefill_async(kvrt_ctx *c, int32_t layer, int32_t n, const int32
     a.n_ksplit = 1;
     const int64_t want = ksplit_env > 0 ? ksplit_env : std::min<int64_t>(256 / wgs(rw), block_keys / min_keys);
     const int nks = (int)std::min<int64_t>(want, 16);
-    if (nks > 1 && (ksplit_env > 0 || block_keys * (nks - 1) / nks >= split_keys)) {
+    if (nks > 1 && !a.short_heads && (ksplit_env > 0 || block_keys * (nks - 1) / nks >= split_keys)) {
         const size_t po = ((size_t)n * hq * qn * nks * D + 63) / 64 * 64;
         const size_t bytes = po * 4 + (size_t)n * hq * qn * nks * 8 + 256;
         hipStreamCaptureStatus st = hipStreamCaptureStatusNone;

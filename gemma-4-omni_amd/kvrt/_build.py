@@ -26,7 +26,7 @@ CSRC = PKG_DIR.parent / "csrc"
 INCLUDE = PKG_DIR.parent.parent / "include"
 LIB_PATH = PKG_DIR / "libkvrt.so"
 CALLS_PATH = PKG_DIR / "kvrt_pycall.so"
-SOURCES = ("kvrt_kernels.hip", "kvrt_prefill.hip", "kvrt_prefill_wide.hip", "kvrt_runtime.hip")
+SOURCES = ("kvrt_kernels.hip", "kvrt_prefill.hip", "kvrt_prefill_wide.hip", "kvrt_prefill_short.hip", "kvrt_runtime.hip")
 
 AGPR_SOURCES = ("kvrt_prefill_wide.hip",)
 

@@ -76,17 +76,16 @@ def _check(rt, orc, q, scale, prefill=True):
         # workgroups and the partials merged (8 and 2 key ranges)
         (8, 1, 512, 0, "contig", [2000, 900], 64),
         (4, 2, 128, 600, "paged", [1500], 40),
-        # the talker's whole-response prefill: a grid of 1024 workgroups, one
-        # wave per head (LDS DMA ring, two waves per workgroup)
+        # the talker's whole-response prefill: two row blocks x two key parts
         (16, 8, 128, 0, "contig", [0, 0, 0, 0], 512),
-        # LDS DMA ring over a wrapped ring layout, two waves per head
+        # a wrapped ring layout, GQA groups of 4
         (8, 2, 128, 200, "ring", [900, 64], 77),
-        # talker-sized grids (>= 512 workgroups, DMA ring): an odd block count
-        # over ragged prefixes, and a windowed ring layout
+        # talker-sized grids: an odd block count over ragged prefixes, and a
+        # windowed ring layout
         (16, 8, 128, 0, "contig", [0, 37, 300, 5], 481),
         (16, 8, 128, 200, "ring", [0, 900, 64, 10], 300),
-        # GQA groups of 6 and 3 (3 q heads per workgroup: the index splits
-        # by a divisor that is not a power of two)
+        # GQA groups of 6 and 3 (index splits by a divisor that is not a power
+        # of two)
         (6, 1, 128, 0, "contig", [100, 37], 50),
         (12, 2, 256, 512, "ring", [300], 40),
         (3, 1, 64, 0, "paged", [70], 33),
@@ -320,3 +319,81 @@ def test_nan_stays_nan_with_and_without_a_key_split(d, hq, hkv, prefix, qn, wind
     out = rt.attend_prefill(0, q.cuda(), [0], 1.0 / math.sqrt(d))
     assert rt.counters()["launches"] == launches + (2 if split else 1)
     assert torch.equal(out.isnan().cpu(), want)
+
+
+def _sampled(hq, hkv, d, window, layout, lens, qn, mask=0):
+    """A chunk of qn queries over sessions of lens rows against the oracle: every
+    q head of the first, the last and 8 other query rows of each."""
+    import random
+
+    from kvrt import KVRuntime, LayerSpec
+
+    gen = torch.Generator().manual_seed(qn + d + lens[0])
+    r = random.Random(qn * 7 + d)
+    ring = dict(ring_rows=window + qn - 1) if layout == "ring" else {}
+    rt = KVRuntime([LayerSpec(kv_heads=hkv, head_dim=d, layout=layout, window=window, **ring)], len(lens),
+                   max(lens) + 8, max_q=qn, device="cuda", pool_seed=3,
+                   pool_pages=sum(n // 16 + 2 for n in lens) if layout == "paged" else 0)
+    ks, vs, hide = [], [], None
+    for s, n in enumerate(lens):
+        k, v = randn_bf16(gen, (1, hkv, n, d)), randn_bf16(gen, (1, hkv, n, d))
+        rt.import_(s, 0, k.cuda(), v.cuda())
+        ks.append(to_np(k[0]))
+        vs.append(to_np(v[0]))
+    if mask:
+        hide = (torch.rand(mask, generator=gen) < 0.5).to(torch.int64)
+        hide[0] = 1  # every query sees a key
+        for s in range(len(lens)):
+            rt.set_prefix_attention(s, hide)
+    q = randn_bf16(gen, (len(lens), hq, qn, d), 0.5)
+    out = rt.attend_prefill(0, q.cuda(), list(range(len(lens))), 1.0 / math.sqrt(d))
+    torch.cuda.synchronize()
+    assert rt.health() == 0
+    for s, n in enumerate(lens):
+        rows = sorted({0, qn - 1, *r.sample(range(qn), min(qn, 8))})
+        for i in rows:
+            pos = n - qn + i
+            seen = np.arange(max(0, pos - window + 1) if window else 0, pos + 1)
+            if hide is not None:
+                seen = seen[(seen >= mask) | (hide.numpy()[np.minimum(seen, mask - 1)] != 0)]
+            ref = O.attend(to_np(q[s])[:, i:i + 1], ks[s][:, seen], vs[s][:, seen], np.array([len(seen) - 1]),
+                           1.0 / math.sqrt(d), 0)
+            assert float(np.abs(to_np(out[s])[:, i:i + 1] - ref).max()) <= ATOL, (s, i)
+
+
+@pytest.mark.parametrize("hq,hkv,d,window,layout,lens,qn,mask", [
+    # four row blocks, one key part: many key blocks, every layout, a prefix mask
+    (16, 8, 128, 0, "contig", [1000, 1100, 1000, 1013], 1000, 0), (16, 8, 128, 300, "ring", [1000] * 4, 1000, 0),
+    (16, 8, 128, 0, "paged", [1000, 1003, 1100, 1000], 1000, 0), (16, 8, 128, 0, "contig", [1000] * 4, 1000, 200),
+    (16, 8, 64, 0, "contig", [1200] * 4, 1200, 0), (16, 8, 64, 200, "ring", [1200] * 4, 1200, 0),
+    (16, 8, 64, 0, "paged", [1200] * 4, 1200, 77),
+    (8, 1, 256, 512, "ring", [1200] * 3, 1200, 0), (8, 1, 256, 0, "contig", [1400, 1500, 1400, 1400], 1400, 90),
+    (8, 1, 256, 0, "paged", [1400] * 4, 1400, 0),
+    # two row blocks x four key parts
+    (16, 8, 128, 0, "contig", [947, 900, 800], 274, 0), (16, 8, 128, 700, "ring", [1500, 947, 800], 274, 0),
+    (16, 8, 128, 0, "paged", [300, 217], 40, 150), (8, 2, 64, 0, "paged", [300, 217], 40, 0),
+    # two x two, and one x four with a key split
+    (16, 8, 64, 0, "contig", [300, 333, 400, 420], 300, 0), (16, 8, 64, 150, "ring", [700] * 4, 300, 0),
+    (16, 8, 128, 0, "contig", [700, 2000], 24, 120), (16, 8, 64, 0, "contig", [700], 24, 0),
+    # PAGED over few keys: one part, then two
+    (16, 8, 128, 0, "paged", [32, 13], 12, 0), (8, 2, 64, 0, "paged", [33, 160], 20, 30),
+])
+def test_prefill_launch_shapes(hq, hkv, d, window, layout, lens, qn, mask):
+    _sampled(hq, hkv, d, window, layout, lens, qn, mask)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("hq,hkv,window,layout,lens,qn,mask", [
+    # tiles of 16 queries x 32 keys: one short, full, one over; 1 to 4 heads per
+    # workgroup and groups of 5 and 6; rings that have wrapped; prefix masks
+    (8, 4, 0, "contig", [15, 31], 15, 0), (8, 4, 0, "contig", [16, 32], 16, 0), (8, 4, 0, "contig", [17, 33], 17, 0),
+    (4, 4, 0, "contig", [65, 96, 97], 40, 0), (16, 8, 0, "contig", [128, 150, 129], 33, 70),
+    (6, 2, 0, "contig", [100, 64], 50, 20), (5, 1, 0, "contig", [60], 9, 0), (6, 1, 0, "contig", [64, 33], 20, 0),
+    (8, 2, 0, "contig", [64, 50], 31, 31), (16, 8, 40, "ring", [900, 70], 50, 0), (8, 8, 100, "ring", [150, 333], 18, 60),
+    (6, 2, 33, "ring", [500, 45], 45, 0), (16, 8, 0, "contig", [300, 310, 290, 305], 200, 100),
+    # two query blocks on the same tiles: 1, 2, 3 and 4 heads
+    (8, 8, 0, "contig", [320] * 4, 300, 0), (16, 8, 0, "contig", [150] * 8, 140, 64), (16, 8, 64, "ring", [500] * 8, 140, 0),
+    (24, 8, 0, "contig", [170] * 8, 170, 0), (32, 8, 0, "contig", [150] * 8, 150, 33),
+])
+def test_prefill_over_few_keys(d, hq, hkv, window, layout, lens, qn, mask):
+    _sampled(hq, hkv, d, window, layout, lens, qn, mask)

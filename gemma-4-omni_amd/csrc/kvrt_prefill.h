@@ -294,25 +294,15 @@ __global__ __launch_bounds__(64 * RW * KS) void prefill_kernel(PrefillArgs a) {
         }
     };
 
-    // At head_dim 256 the first V blocks are fetched with the first K blocks, a
-    // round trip earlier than beside the first K Q^T (Q 9 over 9 6.9 -> 6.6 us).
-    // At 512 that would hold the first scores up by 32 KiB more, and below, where
-    // several workgroups share a CU, it is no faster.
-    constexpr bool V_FIRST = D == 256;
     Fetch kf{}, vf{};
-    // Parts with a block in the range; the others fetch nothing ahead of the
-    // loop and add nothing at its end.
+    // parts with a block in the range; the others fetch no first K block and
+    // add nothing at the end
     const int nparts = KS == 1 ? 1 : max(1, min(KS, (kend - kstart + kPfKeys - 1) / kPfKeys));
-    if (ngroups > 0) {  // the first K and V blocks
+    if (ngroups > 0) {  // the first K blocks
         kf = next_fetch();
-        vf = kf;
-        if (part < nparts) {
+        if (part < nparts)
 #pragma unroll
             for (int i = 0; i < IPW; ++i) fetch(std::false_type{}, kf, 0, i);
-            if constexpr (V_FIRST)
-#pragma unroll
-                for (int i = 0; i < IPW; ++i) fetch(std::true_type{}, vf, 0, i);
-        }
     }
 
     // A negative scale is moved into q's sign bits (exact, below), so that the
@@ -357,12 +347,13 @@ __global__ __launch_bounds__(64 * RW * KS) void prefill_kernel(PrefillArgs a) {
     f32x16_t s;         // scores of the block after it
     int cur = 0;  // the iteration
     // The iteration's DMAs (the K blocks of group it + 2, then the V blocks of
-    // it + 1), spread over SPAN steps: those of K Q^T, at head_dim 512 the first
-    // half of the P V ones, whose MFMAs leave the most issue slots free. Past
-    // the last group they read its last key (a branch around each costs more
-    // than the DMAs it would save); up to head_dim 256 the last iteration, which
-    // has no K Q^T, issues none, and the kernel's end waits for none.
-    constexpr int DMA0 = D == 512 ? NK : 0, SPAN = D == 512 ? NP / 2 : NK;
+    // it + 1), spread over SPAN steps: up to head_dim 128 those of K Q^T, at 256
+    // the first half of all (59 against 61 us over 2339 cold keys), at 512 of the
+    // P V ones, whose MFMAs leave the most issue slots free. Past the last group
+    // they read its last key (a branch around each costs more than the DMAs it
+    // would save), but the last iteration skips those of K Q^T, and up to
+    // head_dim 128 the kernel's end waits for none.
+    constexpr int DMA0 = D == 512 ? NK : 0, SPAN = D == 512 ? NP / 2 : D == 256 ? (NK + NP) / 2 : NK;
     auto dma_at = [&](auto c_c) __attribute__((always_inline)) {
         constexpr int c = decltype(c_c)::value - DMA0;
         if constexpr (c >= 0 && c < SPAN)
@@ -514,11 +505,11 @@ __global__ __launch_bounds__(64 * RW * KS) void prefill_kernel(PrefillArgs a) {
             x = make_uint4(x.x ^ flip, x.y ^ flip, x.z ^ flip, x.w ^ flip);
             asm volatile("" : "+v"(x.x), "+v"(x.y), "+v"(x.z), "+v"(x.w));
         }
-        // the second K blocks, in flight beside the first K Q^T
-        if constexpr (!V_FIRST)
+        // the first V blocks and the second K blocks, in flight beside the first K Q^T
+        vf = kf;
 #pragma unroll
-            for (int i = 0; i < IPW; ++i) fetch(std::true_type{}, vf, 0, i);
-        if (ngroups > 1) {
+        for (int i = 0; i < IPW; ++i) fetch(std::true_type{}, vf, 0, i);
+        if (D >= 256 || ngroups > 1) {  // (D 512, Q 24 over 49: 14.5 us with the test, 14.2 without)
             kf = next_fetch();
 #pragma unroll
             for (int i = 0; i < IPW; ++i) fetch(std::false_type{}, kf, 1, i);

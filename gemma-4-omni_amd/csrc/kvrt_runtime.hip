@@ -354,17 +354,31 @@ int min_keys_per_wave(int keys_per_iter) {
 #endif
 constexpr int64_t kSplitKeyBucket = KVRT_SPLIT_KEY_BUCKET;
 // Whether a decode merges its workgroup partials in its last workgroup
-// (kvrt_config.decode_merge) instead of a second kernel. AUTO: when the
-// partials of one (item, kv head) total at most KVRT_SINGLE_LAUNCH_BYTES
-// (12 KiB): the merging workgroup reads them all, three dependent memory
-// round trips after the last partial lands, which costs about what the merge
-// kernel's launch does; beyond that one workgroup's read takes longer. (2 query
-// rows at D 128: 8 KiB 16.2 us in one launch, 17.3 in two; 16 KiB 9.6 and 8.1,
-// 24 KiB 9.7 and 8.2, 32 KiB 10.6 and 8.5.)
-bool single_launch_decode(int mode, bool mfma, int head_dim, int R, int rows, int n_parts) {
+// (kvrt_config.decode_merge) instead of a second kernel. AUTO: one partial, or
+// when those of one (item, kv head) total at most KVRT_SINGLE_LAUNCH_BYTES (12
+// KiB); in an eager call of at most 16 partials (up to which both merges round
+// alike, so that the result does not depend on the capture) up to 24 KiB, on
+// the MFMA kernel 32 KiB. The merging workgroup reads them all, three dependent
+// memory round trips after the last partial lands; the merge kernel costs up to
+// 0.7 us in a graph replay but a launch in an eager call: 2.5 us of host time,
+// 1.6 us on a full queue. us in one launch and in two, one stream of 8 KV heads
+// unless said otherwise, (query rows) x (head_dim):
+//   graph: 8 KiB 16.2, 17.3; 16 KiB (2 x 128, 4 streams) 11.6, 10.8; 18 KiB 8.2,
+//     7.3; 30 KiB 10.1, 8.0; 32 KiB (8 x 128, one KV head) 7.1, 6.4
+//   eager, VALU: 16 KiB 11.8, 12.0 (listener 4 x 1500: 412, 430 us a frame); 24
+//     KiB (4 x 128, talker masks) 9.1, 10.6, 4 streams 11.9, 12.6; 32 KiB 15.9,
+//     15.3; 18 KiB in 18 partials 8.4, 9.2, two streams 10.8, 10.2; 30 in 30
+//     13.5, 10.9
+//   eager, MFMA, one KV head: 32 KiB (8 x 128, 400 keys) 7.6, 9.1; (8 x 256, 130
+//     keys) 8.0, 9.4
+bool single_launch_decode(int mode, bool mfma, int head_dim, int R, int rows, int n_parts, hipStream_t st) {
     static const int limit = env_int("KVRT_SINGLE_LAUNCH_BYTES", 12288);
     if (mode == KVRT_MERGE_SEPARATE || !(mfma || decode_wg_merge(head_dim, R))) return false;
-    return mode == KVRT_MERGE_LAST_WG || (int64_t)n_parts * rows * head_dim * 4 <= limit;
+    const int64_t bytes = (int64_t)n_parts * rows * head_dim * 4;
+    if (mode == KVRT_MERGE_LAST_WG || n_parts == 1 || bytes <= limit) return true;
+    if (n_parts > 16 || bytes > (mfma ? (int64_t)limit * 8 / 3 : (int64_t)limit * 2)) return false;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(st, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone;
 }
 
 int choose_splits(int target, int n_items, int kv_heads, int64_t max_keys, int keys_per_iter) {
@@ -833,7 +847,7 @@ int decode_impl(kvrt_ctx *c, int layer, int n, const int32_t *slots, const kvrt_
     a.n_split = n_split;
     a.advance = fused ? 1 : 0;
     a.n_parts = (mfma || decode_wg_merge(D, R)) ? n_split / kWaves : n_split;
-    a.cnt = single_launch_decode(c->cfg.decode_merge, mfma, D, R, rows, a.n_parts) ? c->d_cnt : nullptr;
+    a.cnt = single_launch_decode(c->cfg.decode_merge, mfma, D, R, rows, a.n_parts, c->stream) ? c->d_cnt : nullptr;
     a.pmask = pmask;
     a.scale_log2 = scale * 1.4426950408889634f;
     for (int i = 0; i < n; ++i) a.slots[i] = slots[i];
@@ -986,7 +1000,6 @@ struct TensorCall {
     PrefixPackArgs pk{};
     bool masked = false;
     bool mfma = false;
-    bool single = false;  // the decode may merge its own partials (bit-identical to the merge kernel)
     int D = 0, rows = 0;
     size_t acc_elems = 0;
     size_t bytes = 0;
@@ -1050,10 +1063,6 @@ int tensor_call_setup(const kvrt_tensor *q, const kvrt_tensor *k, const kvrt_ten
     tc.rows = rows;
     tc.acc_elems = (size_t)n * hkv * a.n_split * Rw * D;
     tc.bytes = (kTensorWsParts + tc.acc_elems + 64) * 4 + (size_t)n * hkv * a.n_split * Rw * 8;
-    // At most 16 partials per (item, kv head): the last workgroup's merge
-    // rounds exactly as the merge kernel's, so the result does not depend on
-    // which of the two ran.
-    tc.single = a.n_parts <= 16 && single_launch_decode(KVRT_MERGE_AUTO, tc.mfma, (int)D, R, rows, a.n_parts);
     return KVRT_OK;
 }
 
@@ -1080,7 +1089,12 @@ int scratch_pointer(int dev, float **out) {
 int tensor_call_launch(TensorCall &tc, float *ws, hipStream_t st, bool single) {
     DecodeArgs &a = tc.a;
     a.err = reinterpret_cast<int32_t *>(ws);
-    a.cnt = single && tc.single ? reinterpret_cast<uint32_t *>(ws + kTensorWsHead + kTensorWsMasks) : nullptr;
+    // At most 16 partials per (item, kv head): the last workgroup's merge
+    // rounds exactly as the merge kernel's, so the result does not depend on
+    // which of the two ran.
+    single = single && a.n_parts <= 16 &&
+             single_launch_decode(KVRT_MERGE_AUTO, tc.mfma, tc.D, rows_tile(tc.rows), tc.rows, a.n_parts, st);
+    a.cnt = single ? reinterpret_cast<uint32_t *>(ws + kTensorWsHead + kTensorWsMasks) : nullptr;
     a.part_acc = ws + kTensorWsParts;
     a.part_ml = reinterpret_cast<float2 *>(a.part_acc + ((tc.acc_elems + 63) / 64) * 64);
     if (tc.masked) {

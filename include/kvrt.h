@@ -158,8 +158,9 @@ typedef struct kvrt_config {
  * LAST_WG: the last workgroup of each (slot, kv head) to finish merges them
  *   inside the decode launch (one launch per layer); the VALU kernel's
  *   16-row tiles at head_dim 512 (no workgroup partials) always use SEPARATE;
- * AUTO: LAST_WG when a (slot, kv head) has at most 12 KiB of partials (one
- *   workgroup reads them all), SEPARATE otherwise.
+ * AUTO: LAST_WG when a (slot, kv head) has one partial, at most 12 KiB of them
+ *   (one workgroup reads them all) or, in a call that is not captured, at most
+ *   24 KiB (MFMA kernel 32) in up to 16; SEPARATE otherwise.
  * Every mode gives the same results, bit for bit, when a (slot, kv head) has
  * at most 16 partial workgroups; beyond that the merge order differs. */
 #define KVRT_MERGE_AUTO 0

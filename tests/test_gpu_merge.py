@@ -175,3 +175,48 @@ def _runtime_layers(specs, n, capacity, merge):
     from kvrt import KVRuntime
 
     return KVRuntime(specs, n, capacity, max_q=1, decode_wgs=192, decode_merge=merge, device="cuda")
+
+
+@pytest.mark.parametrize("hq,hkv,d,keys,n,eager,captured", [
+    (16, 8, 128, 1000, 4, 1, 2),  # VALU, 16 partials of 1 KiB
+    (4, 2, 256, 200, 2, 1, 2),    # VALU, 8 partials of 2 KiB
+    (4, 2, 256, 1000, 2, 2, 2),   # VALU, 16 partials of 2 KiB
+    (8, 8, 128, 600, 2, 1, 1),    # VALU, 10 partials of 512 B
+    (8, 1, 256, 130, 1, 1, 2),    # MFMA, 4 partials of 8 KiB
+    (8, 2, 128, 700, 1, 1, 2),    # MFMA, 12 partials of 2 KiB
+    (16, 8, 128, 2200, 1, 2, 2),  # MFMA, more than 16 partials
+    (8, 1, 512, 40, 1, 1, 2),     # MFMA, 2 partials of 16 KiB
+    (8, 1, 256, 400, 1, 2, 2),    # 7 partials of 8 KiB
+])
+def test_auto_by_capture_gives_the_same_bits(hq, hkv, d, keys, n, eager, captured):
+    """A launch costs an eager call more than a graph replay, so AUTO merges up
+    to 24 KiB of partials in the launch (MFMA kernel 32) when eager, 12 KiB when captured, and the
+    replays still equal the eager call bit for bit."""
+    from kvrt import KVRuntime, LayerSpec
+
+    gen = torch.Generator().manual_seed(keys + d)
+    rt = KVRuntime([LayerSpec(kv_heads=hkv, head_dim=d)], n, keys + 8, max_q=1, device="cuda")
+    for s in range(n):
+        k, v = randn_bf16(gen, (1, hkv, keys - s, d)).cuda(), randn_bf16(gen, (1, hkv, keys - s, d)).cuda()
+        rt.import_(s, 0, k, v)
+    q = randn_bf16(gen, (n, hq, 1, d)).cuda()
+    slots = list(range(n))
+    before = rt.counters()["launches"]
+    want = rt.attend(0, q, slots, 0.08)
+    assert rt.counters()["launches"] - before == eager
+    rt.synchronize()
+    out = torch.empty_like(q)
+    before = rt.counters()["launches"]
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        rt.attend(0, q, slots, 0.08, out=out)
+    assert rt.counters()["launches"] - before == captured
+    for _ in range(3):
+        out.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        rt.sync_lengths()
+        assert torch.equal(rt.attend(0, q, slots, 0.08), want)
+        rt.synchronize()

@@ -145,12 +145,20 @@ PyObject *guarded(Py_ssize_t nargs, Py_ssize_t want, F body) {
     return PyLong_FromLong(rc);
 }
 
+// The runtime call, the parse done. An exception out of it (its vectors can
+// fail to allocate) is a device error and not the general path's to repeat: the
+// call may have mapped pages or enqueued work. The interpreter lock is held
+// again before anything else runs.
 template <class F>
 long without_gil(F call) {
     long rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = call();
-    Py_END_ALLOW_THREADS
+    PyThreadState *const thread = PyEval_SaveThread();
+    try {
+        rc = call();
+    } catch (...) {
+        rc = KVRT_EDEVICE;
+    }
+    PyEval_RestoreThread(thread);
     return rc;
 }
 

@@ -497,6 +497,7 @@ class KVRuntime:
         shared layers' entries are ignored) and set its prefix mask. Returns
         the slot's generation. Mirrors gemma4_listener_batch_import_cache_async
         (gemma4_listener_microbatch_impl.inc:2590-2640)."""
+        layers = list(layers)  # walked more than once
         descs = self._session_descs(layers)
         if descs is not None:
             self._bind()

@@ -279,3 +279,36 @@ def test_talker_mask_validation(kwargs, ok):
     else:
         with pytest.raises(ValueError):
             TalkerMask(**args)
+
+
+def test_import_session_takes_any_iterable_of_layers():
+    """The layers of a session as a list, a zip or a generator: each is walked
+    once, and every layer reaches its import."""
+    from kvrt import KVRuntime, LayerSpec
+
+    class Runtime:
+        layers = [LayerSpec(kv_heads=1, head_dim=64)] * 2 + [LayerSpec(kv_heads=1, head_dim=64, shared_src=0)]
+        _session_descs = KVRuntime._session_descs
+        import_session = KVRuntime.import_session
+
+        def __init__(self):
+            self.seen = []
+
+        def _owner(self, i):
+            return 0 if i == 2 else i
+
+        def reset_slot(self, slot):
+            self.seen.append(("reset", slot))
+
+        def import_(self, slot, layer, k, v):
+            self.seen.append((slot, layer, k, v))
+
+        def slot_generation(self, slot):
+            return 7
+
+    ks, vs = ([torch.zeros(1, 1, 4, 64, dtype=torch.bfloat16) for _ in range(3)] for _ in range(2))
+    for layers in (list(zip(ks, vs)), zip(ks, vs), ((k, v) for k, v in zip(ks, vs))):
+        rt = Runtime()
+        assert rt.import_session(3, layers) == 7
+        assert [x[:2] for x in rt.seen] == [("reset", 3), (3, 0), (3, 1)]
+        assert all(x[2] is ks[x[1]] and x[3] is vs[x[1]] for x in rt.seen[1:])

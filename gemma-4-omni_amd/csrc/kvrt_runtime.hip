@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "kvrt_internal.h"
+#include "kvrt_range.h"
 
 using namespace kvrt;
 
@@ -2099,8 +2100,7 @@ int kvrt_attend_prefill_async(kvrt_ctx *c, int32_t layer, int32_t n, const int32
         if (out->dims[i] != q->dims[i]) return KVRT_EINVAL;
     const int group = (int)(hq / hkv);
     if (!std::isfinite(scale)) return KVRT_EINVAL;
-    uint64_t tile_keys = 0;
-    int64_t block_keys = 0;  // most keys any 16-query block sees
+    int64_t block_keys = 0;  // most keys any 16 queries see
     for (int i = 0; i < n; ++i) {
         const int L = c->len_at(slots[i], layer);
         if (L < qn) return KVRT_ESTATE;
@@ -2112,7 +2112,6 @@ int kvrt_attend_prefill_async(kvrt_ctx *c, int32_t layer, int32_t n, const int32
         for (int64_t q0 = 0; q0 < qn; q0 += 16) {
             const int64_t kend = L - qn + std::min<int64_t>(qn, q0 + 16);
             const int64_t kstart = s.window > 0 ? std::max<int64_t>(0, L - qn + q0 - s.window + 1) : 0;
-            tile_keys += (uint64_t)(kend - kstart);
             block_keys = std::max<int64_t>(block_keys, kend - kstart);
         }
     }
@@ -2233,8 +2232,19 @@ int kvrt_attend_prefill_async(kvrt_ctx *c, int32_t layer, int32_t n, const int32
     for (int i = 0; i < n; ++i) a.slots[i] = slots[i];
     c->counters.launches += a.n_ksplit > 1 ? 2 : 1;
     if (launch_prefill(a, D, enq(c)) != hipSuccess) return poison(c);
-    c->counters.attended_keys += tile_keys * hkv;
-    c->counters.attended_bytes += tile_keys * hkv * (uint64_t)D * 2 * 2;
+    // keys its workgroups read: those of 32 rw rows, or of rw 16-query blocks by short_heads heads
+    const int64_t wg_rows = a.short_heads ? 16 * rw : 32 * rw, per_query = a.short_heads ? 1 : group;
+    uint64_t keys = 0;
+    for (int i = 0; i < n; ++i)
+        for (int64_t r0 = 0; r0 < qn * per_query; r0 += wg_rows) {
+            const int64_t last = std::min(qn * per_query, r0 + wg_rows) - 1;
+            const KeyRange r = prefill_range((int)(c->len_at(slots[i], layer) - qn), (int)(r0 / per_query),
+                                             (int)(last / per_query), s.window, 1, 0, kPfKeys);
+            keys += (uint64_t)(r.kend - r.kstart);
+        }
+    keys *= (uint64_t)hkv * (a.short_heads ? group / a.short_heads : 1);
+    c->counters.attended_keys += keys;
+    c->counters.attended_bytes += keys * (uint64_t)D * 2 * 2;
     return KVRT_OK;
 }
 

@@ -180,8 +180,9 @@ typedef struct kvrt_counters {
     uint64_t launches;
     uint64_t appended_rows;     /* token rows appended (sum over slots, layers) */
     uint64_t appended_bytes;    /* K+V payload bytes written by append          */
-    uint64_t attended_keys;     /* visible keys read by attention (per kv head) */
-    uint64_t attended_bytes;    /* K+V bytes read by attention                  */
+    uint64_t attended_keys;     /* keys read by attention, times kv heads (a chunk:
+                                   by every workgroup that reads them)          */
+    uint64_t attended_bytes;    /* their K+V bytes                              */
     uint64_t gathered_bytes;    /* bytes written by gather (incl. padding)      */
     uint64_t truncations;
     uint64_t truncated_rows;

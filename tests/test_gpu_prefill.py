@@ -397,3 +397,19 @@ def test_prefill_launch_shapes(hq, hkv, d, window, layout, lens, qn, mask):
 ])
 def test_prefill_over_few_keys(d, hq, hkv, window, layout, lens, qn, mask):
     _sampled(hq, hkv, d, window, layout, lens, qn, mask)
+
+
+@pytest.mark.parametrize("hq,hkv,d,window,layout,n_rows,qn,keys", [
+    # four 32-row blocks per workgroup: 64 queries of 2 heads, 128 of one, 16 of 8
+    (2, 1, 512, 0, "contig", 300, 100, 264 + 300), (1, 1, 512, 0, "contig", 300, 130, 298 + 300),
+    (8, 1, 512, 40, "contig", 500, 20, (39 + 16) + (39 + 4)),
+    # 16-query blocks, four and two heads per workgroup
+    (4, 1, 128, 0, "contig", 60, 20, 56 + 60), (8, 4, 128, 0, "contig", 60, 20, 4 * (56 + 60)),
+])
+def test_attended_counters_are_the_rows_read(hq, hkv, d, window, layout, n_rows, qn, keys):
+    rt, _, q = _setup(hq, hkv, d, window, layout, [n_rows - qn], qn, seed=1)
+    before = rt.counters()
+    rt.attend_prefill(0, q.cuda(), [0], 0.1)
+    after = rt.counters()
+    assert after["attended_keys"] - before["attended_keys"] == keys
+    assert after["attended_bytes"] - before["attended_bytes"] == keys * d * 4

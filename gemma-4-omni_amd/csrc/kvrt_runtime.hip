@@ -287,11 +287,14 @@ constexpr int kMaxWgPerHead = 64;
 // step waits for every one of them, run on the MFMA kernel too (8 rows, D 256
 // x 512 ring keys: 9.3 -> 7.5 us with the merge; D 128 x 130 9.5 -> 6.5; 4
 // rows, D 128 x 513 7.6 -> 6.5; but 4 rows at D 256 x 33 7.3 and 7.4, 2 rows
-// at D 64 x 1100 5.9 and 6.2). Short batches stay on the VALU kernel, which
-// kvrt_counters.mfma_decodes reports of them: 10.3 against 8.0 us with 4
-// streams of that ring, and 0.7 % of a two-model step. `keys` is the launch's
-// key count rounded up to the split bucket, so the choice, like the split
-// count, stays fixed within a bucket.
+// at D 64 x 1100 5.9 and 6.2; a step of one thinker and one talker stream on
+// two streams 393 -> 379 us at 4096 positions, 384 -> 355 at 1024). P is two
+// bf16 terms there and fp32 on the VALU kernel; the error against float64 is
+// the same to six digits (160 shapes of 24 to 2000 keys: that of rounding the
+// output). Batches stay on the VALU kernel: alone they would gain (4 streams of
+// that ring 10.3 -> 8.0 us), beside a talker's launches a step lost 0.7 %.
+// `keys` is the launch's key count rounded up to the split bucket, so the
+// choice, like the split count, stays fixed within a bucket.
 constexpr int64_t kMfmaDecodeMinKeys8 = 2048;
 bool use_mfma_decode(int mode, int dtype, int rows_tile_, int head_dim, int64_t keys, int layout, int n_items) {
     if (mode == KVRT_DECODE_VALU) return false;
@@ -359,11 +362,13 @@ constexpr int64_t kSplitKeyBucket = KVRT_SPLIT_KEY_BUCKET;
 // when those of one (item, kv head) total at most KVRT_SINGLE_LAUNCH_BYTES (12
 // KiB); in an eager call of at most 16 partials (up to which both merges round
 // alike, so that the result does not depend on the capture) up to 24 KiB, on
-// the MFMA kernel 32 KiB. The merging workgroup reads them all, three dependent
-// memory round trips after the last partial lands; the merge kernel costs up to
-// 0.7 us in a graph replay but a launch in an eager call: 2.5 us of host time,
-// 1.6 us on a full queue. us in one launch and in two, one stream of 8 KV heads
-// unless said otherwise, (query rows) x (head_dim):
+// the MFMA kernel 32 KiB; and always up to 32 KiB where the context's launches
+// run beside another model's (decode_wgs set). The merging workgroup reads them
+// all, three dependent memory round trips after the last partial lands; the
+// merge kernel costs up to 0.7 us in a graph replay alone but a launch in an
+// eager call: 2.5 us of host time, 1.6 us on a full queue; and in replays on two
+// streams the launches of one delay the other's. us in one launch and in two,
+// one stream of 8 KV heads unless said otherwise, (query rows) x (head_dim):
 //   graph: 8 KiB 16.2, 17.3; 16 KiB (2 x 128, 4 streams) 11.6, 10.8; 18 KiB 8.2,
 //     7.3; 30 KiB 10.1, 8.0; 32 KiB (8 x 128, one KV head) 7.1, 6.4
 //   eager, VALU: 16 KiB 11.8, 12.0 (listener 4 x 1500: 412, 430 us a frame); 24
@@ -372,12 +377,14 @@ constexpr int64_t kSplitKeyBucket = KVRT_SPLIT_KEY_BUCKET;
 //     13.5, 10.9
 //   eager, MFMA, one KV head: 32 KiB (8 x 128, 400 keys) 7.6, 9.1; (8 x 256, 130
 //     keys) 8.0, 9.4
-bool single_launch_decode(int mode, bool mfma, int head_dim, int R, int rows, int n_parts, hipStream_t st) {
+//   a step of one thinker and one talker stream on two streams, talker partials
+//     18 KiB (1024 positions) 355, 430; 28 KiB (4096) 379, 461
+bool single_launch_decode(int mode, bool mfma, int head_dim, int R, int rows, int n_parts, bool beside, hipStream_t st) {
     static const int limit = env_int("KVRT_SINGLE_LAUNCH_BYTES", 12288);
     if (mode == KVRT_MERGE_SEPARATE || !(mfma || decode_wg_merge(head_dim, R))) return false;
-    const int64_t bytes = (int64_t)n_parts * rows * head_dim * 4;
-    if (mode == KVRT_MERGE_LAST_WG || n_parts == 1 || bytes <= limit) return true;
-    if (n_parts > 16 || bytes > (mfma ? (int64_t)limit * 8 / 3 : (int64_t)limit * 2)) return false;
+    const int64_t bytes = (int64_t)n_parts * rows * head_dim * 4, most = (int64_t)limit * 8 / 3;
+    if (mode == KVRT_MERGE_LAST_WG || n_parts == 1 || bytes <= (beside ? most : limit)) return true;
+    if (n_parts > 16 || bytes > (mfma ? most : (int64_t)limit * 2)) return false;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     return hipStreamIsCapturing(st, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone;
 }
@@ -848,7 +855,9 @@ int decode_impl(kvrt_ctx *c, int layer, int n, const int32_t *slots, const kvrt_
     a.n_split = n_split;
     a.advance = fused ? 1 : 0;
     a.n_parts = (mfma || decode_wg_merge(D, R)) ? n_split / kWaves : n_split;
-    a.cnt = single_launch_decode(c->cfg.decode_merge, mfma, D, R, rows, a.n_parts, c->stream) ? c->d_cnt : nullptr;
+    a.cnt = single_launch_decode(c->cfg.decode_merge, mfma, D, R, rows, a.n_parts, c->cfg.decode_wgs > 0, c->stream)
+                ? c->d_cnt
+                : nullptr;
     a.pmask = pmask;
     a.scale_log2 = scale * 1.4426950408889634f;
     for (int i = 0; i < n; ++i) a.slots[i] = slots[i];
@@ -1094,7 +1103,7 @@ int tensor_call_launch(TensorCall &tc, float *ws, hipStream_t st, bool single) {
     // rounds exactly as the merge kernel's, so the result does not depend on
     // which of the two ran.
     single = single && a.n_parts <= 16 &&
-             single_launch_decode(KVRT_MERGE_AUTO, tc.mfma, tc.D, rows_tile(tc.rows), tc.rows, a.n_parts, st);
+             single_launch_decode(KVRT_MERGE_AUTO, tc.mfma, tc.D, rows_tile(tc.rows), tc.rows, a.n_parts, false, st);
     a.cnt = single ? reinterpret_cast<uint32_t *>(ws + kTensorWsHead + kTensorWsMasks) : nullptr;
     a.part_acc = ws + kTensorWsParts;
     a.part_ml = reinterpret_cast<float2 *>(a.part_acc + ((tc.acc_elems + 63) / 64) * 64);

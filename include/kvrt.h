@@ -134,7 +134,9 @@ typedef struct kvrt_config {
                              (0 = 512, or KVRT_TARGET_WGS; int8 twice that,
                              the bf16 MFMA kernel half). Contexts whose
                              launches run beside another model's on a second
-                             stream do better with fewer (e.g. 192)          */
+                             stream do better with fewer (e.g. 192), and with
+                             decode_merge AUTO's wider limit, which a set
+                             value selects                                    */
     int32_t decode_kernel; /* KVRT_DECODE_*: which kernel runs bf16 decodes of
                              8 or 16 query rows per kv head                   */
     int32_t decode_merge;  /* KVRT_MERGE_*: how a split-K decode combines its
@@ -147,7 +149,9 @@ typedef struct kvrt_config {
  * otherwise (int8 included). VALU / MFMA force one kernel for every
  * eligible decode (MFMA: bf16 with 8 or 16 rows per kv head, or int8 PAGED
  * with up to 8; not the talker masks; other decodes always run on the VALU
- * kernel). */
+ * kernel). The MFMA kernels hold the weights of P V as two bf16 terms (2^-17
+ * relative), the VALU kernel in fp32; against float64 both err by the rounding
+ * of the bf16 output. */
 #define KVRT_DECODE_AUTO 0
 #define KVRT_DECODE_VALU 1
 #define KVRT_DECODE_MFMA 2
@@ -160,7 +164,9 @@ typedef struct kvrt_config {
  *   16-row tiles at head_dim 512 (no workgroup partials) always use SEPARATE;
  * AUTO: LAST_WG when a (slot, kv head) has one partial, at most 12 KiB of them
  *   (one workgroup reads them all) or, in a call that is not captured, at most
- *   24 KiB (MFMA kernel 32) in up to 16; SEPARATE otherwise.
+ *   24 KiB (MFMA kernel 32) in up to 16; at most 32 KiB in any call of a
+ *   context with decode_wgs set (its launches run beside another model's);
+ *   SEPARATE otherwise.
  * Every mode gives the same results, bit for bit, when a (slot, kv head) has
  * at most 16 partial workgroups; beyond that the merge order differs. */
 #define KVRT_MERGE_AUTO 0

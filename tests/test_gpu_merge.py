@@ -177,25 +177,26 @@ def _runtime_layers(specs, n, capacity, merge):
     return KVRuntime(specs, n, capacity, max_q=1, decode_wgs=192, decode_merge=merge, device="cuda")
 
 
-@pytest.mark.parametrize("hq,hkv,d,keys,n,eager,captured", [
-    (16, 8, 128, 1000, 4, 1, 2),  # VALU, 16 partials of 1 KiB
-    (4, 2, 256, 200, 2, 1, 2),    # VALU, 8 partials of 2 KiB
-    (4, 2, 256, 1000, 2, 2, 2),   # VALU, 16 partials of 2 KiB
-    (8, 8, 128, 600, 2, 1, 1),    # VALU, 10 partials of 512 B
-    (8, 1, 256, 130, 1, 1, 2),    # MFMA, 4 partials of 8 KiB
-    (8, 2, 128, 700, 1, 1, 2),    # MFMA, 12 partials of 2 KiB
-    (16, 8, 128, 2200, 1, 2, 2),  # MFMA, more than 16 partials
-    (8, 1, 512, 40, 1, 1, 2),     # MFMA, 2 partials of 16 KiB
-    (8, 1, 256, 400, 1, 2, 2),    # 7 partials of 8 KiB
+@pytest.mark.parametrize("hq,hkv,d,keys,n,wgs,eager,captured", [
+    (16, 8, 128, 1000, 4, 0, 1, 2),  # VALU, 16 partials of 1 KiB
+    (4, 2, 256, 200, 2, 0, 1, 2),    # VALU, 8 partials of 2 KiB
+    (4, 2, 256, 1000, 2, 0, 2, 2),   # VALU, 16 partials of 2 KiB
+    (8, 8, 128, 600, 2, 0, 1, 1),    # VALU, 10 partials of 512 B
+    (8, 1, 256, 130, 1, 0, 1, 2),    # MFMA, 4 partials of 8 KiB
+    (8, 2, 128, 700, 1, 0, 1, 2),    # MFMA, 12 partials of 2 KiB
+    (16, 8, 128, 2200, 1, 0, 2, 2),  # MFMA, more than 16 partials
+    (8, 1, 512, 40, 1, 0, 1, 2),     # MFMA, 2 partials of 16 KiB
+    (16, 8, 128, 2200, 1, 224, 1, 1),  # a context beside another's: 28 partials of 1 KiB
+    (8, 1, 256, 400, 1, 0, 2, 2),    # 7 partials of 8 KiB
 ])
-def test_auto_by_capture_gives_the_same_bits(hq, hkv, d, keys, n, eager, captured):
+def test_auto_by_capture_gives_the_same_bits(hq, hkv, d, keys, n, wgs, eager, captured):
     """A launch costs an eager call more than a graph replay, so AUTO merges up
     to 24 KiB of partials in the launch (MFMA kernel 32) when eager, 12 KiB when captured, and the
     replays still equal the eager call bit for bit."""
     from kvrt import KVRuntime, LayerSpec
 
     gen = torch.Generator().manual_seed(keys + d)
-    rt = KVRuntime([LayerSpec(kv_heads=hkv, head_dim=d)], n, keys + 8, max_q=1, device="cuda")
+    rt = KVRuntime([LayerSpec(kv_heads=hkv, head_dim=d)], n, keys + 8, max_q=1, decode_wgs=wgs, device="cuda")
     for s in range(n):
         k, v = randn_bf16(gen, (1, hkv, keys - s, d)).cuda(), randn_bf16(gen, (1, hkv, keys - s, d)).cuda()
         rt.import_(s, 0, k, v)

@@ -358,7 +358,7 @@ struct SlotMoveArgs {
 // layers listed (bf16) is written once, from the imported K / V where a
 // position of [0, rows) lives in it and as zeros elsewhere; their device
 // lengths become rows and the slot's prefix mask is cleared.
-constexpr int kMaxOpenLayers = 48;  // layers per launch (2.7 KB of arguments)
+constexpr int kMaxOpenLayers = 48;  // layers per launch
 struct OpenLayer {
     const uint16_t *k;        // [kv_heads, rows, D], rows head_stride / row_stride elements apart
     const uint16_t *v;
@@ -374,6 +374,7 @@ struct OpenArgs {
     int32_t n_layers;
     OpenLayer l[kMaxOpenLayers];
 };
+static_assert(sizeof(OpenArgs) == 1952, "under 2 KB of launch arguments");
 
 struct CopyRowsArgs {
     const uint8_t *src;

@@ -91,3 +91,29 @@ def test_refusals_are_those_of_the_single_calls():
     with pytest.raises(KVRTError):
         rt.import_session(7, [(ok, ok)])
     assert rt.health() == 0
+
+
+@pytest.mark.parametrize("n_layers", [48, 49, 100])
+def test_more_layers_than_one_launch_takes(n_layers):
+    """48 layers per launch: a topology past them opens in as few launches as
+    hold it, every layer's rows, zeros and lengths in place."""
+    from kvrt import KVRuntime, LayerSpec
+
+    gen = torch.Generator().manual_seed(n_layers)
+    rt = KVRuntime([LayerSpec(kv_heads=1 + l % 3, head_dim=64) for l in range(n_layers)], 2, 24, max_q=1, device="cuda")
+    for l in range(n_layers):
+        for t in rt.storage(l)[:2]:
+            t.normal_()
+    other = [t[0].clone() for l in range(n_layers) for t in rt.storage(l)[:2]]
+    kv = [tuple(randn_bf16(gen, (1, 1 + l % 3, 5 + l % 19, 64)).cuda() for _ in range(2)) for l in range(n_layers)]
+    before = rt.counters()["launches"]
+    rt.import_session(1, kv, None)
+    assert rt.counters()["launches"] - before == (n_layers + 47) // 48
+    rt.sync_lengths()
+    for l in range(n_layers):
+        rows = 5 + l % 19
+        assert rt.seq_length(1, l) == rows
+        for t, src in zip(rt.storage(l)[:2], kv[l]):
+            assert torch.equal(t[1, :, :rows], src[0]) and not t[1, :, rows:].any()
+    assert all(torch.equal(a, b[0]) for a, b in zip(other, (t for l in range(n_layers) for t in rt.storage(l)[:2])))
+    assert rt.health() == 0

@@ -398,7 +398,7 @@ hipError_t launch_decode_talker(const TalkerArgs &a, int head_dim, int rows_per_
 // Chunked-prefill attention on MFMA (bf16 CONTIG / RING / PAGED layers).
 hipError_t launch_prefill(const PrefillArgs &a, int head_dim, hipStream_t s);
 hipError_t launch_prefill_wide(const PrefillArgs &a, int head_dim, hipStream_t s);  // head_dim 256, 512
-hipError_t launch_prefill_short(const PrefillArgs &a, int head_dim, hipStream_t s);  // head_dim 128, few keys
+hipError_t launch_prefill_short(const PrefillArgs &a, int head_dim, hipStream_t s);  // head_dim 64, 128, few keys
 constexpr int kPfKeys = 32;  // keys per staged block of the prefill kernel
 hipError_t launch_set_lens(const SetLenArgs &a, hipStream_t s);
 hipError_t launch_set_pages(int32_t *pt, int n, const int32_t *idx, const int32_t *val,

@@ -1,5 +1,5 @@
-// kvrt_prefill_short.hip — prefill of head_dim 128 over few keys (CONTIG and
-// RING layers): 16-query tiles.
+// kvrt_prefill_short.hip — prefill of head_dim 64 and 128 over few keys (CONTIG
+// and RING layers): 16-query tiles.
 //
 // A wave holds 16 queries of one head, so a 32-key tile is half the MFMA chain
 // and half the softmax of a 32-row block of kvrt_prefill.h, and few rows still
@@ -11,7 +11,7 @@
 // Wave w of a workgroup computes head w % heads over key part (w / heads) % KS
 // of query block w / (heads KS): tile j of 32 keys goes to part j % KS, QB
 // blocks share the staged tiles, and the parts are combined through LDS at the
-// end. Per tile and wave:
+// end. Per tile and wave, at head_dim 128 (half the products at 64):
 //   S^T (32 keys x 16 queries) = K Q^T   8 v_mfma_f32_16x16x32_bf16
 //   online softmax per query (fp32, exp2 domain)
 //   O^T (128 x 16) += V^T P^T            16 v_mfma_f32_16x16x32_bf16 (P in two bf16 terms)
